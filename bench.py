@@ -278,7 +278,10 @@ def describe_variant(shape):
     or the two-step row stream (strips of block columns, chunks of rows)."""
     b, c, v, f = shape
     flags = [name for bit, name in ((1, "nt_store"), (2, "nt_load"), (4, "xcd_rows"), (8, "lane_shuffle"),
-                                    (16, "two_step"), (64, "three_step"), (128, "row_stream")) if f & bit]
+                                    (16, "two_step"), (64, "three_step"), (128, "row_stream"), (256, "n_step")) if f & bit]
+    if f & 256:
+        return {"kernel": "k_phys_stepn", "block": b, "tile_rows": c, "tile_width": v, "flags": flags,
+                "steps_per_launch": f >> 12}
     if f & 64:
         return {"kernel": "k_phys_step3", "block": b, "tile_rows": c, "tile_width": v, "flags": flags,
                 "steps_per_launch": 3}

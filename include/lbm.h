@@ -249,8 +249,14 @@ int lbm_variant_count(void);
  * end with a one-step launch), bit 6 three steps per launch through an LDS
  * tile with a two-cell ring (same conditions; the steps left over run one
  * per launch), bit 7 (with bit 4) the two steps streamed down strips of vec
- * columns in chunks of cells_per_thread rows.  Every variant gives the same
- * bits at every slot a fluid cell can read. */
+ * columns in chunks of cells_per_thread rows, bit 8 the number of steps per
+ * launch in the bits from 12 on, through an LDS tile with a ring of one cell
+ * less than that (nx, ny at least the number of steps; the other conditions
+ * as for bit 6).  Every variant gives the same bits at every slot a fluid
+ * cell can read.  Until a shape is chosen with lbm_set_variant or
+ * lbm_autotune, lbm_run takes a multi-step shape by the lattice's size and
+ * ends with a one-step launch of the shape lbm_get_variant names, so that
+ * both buffers hold what one launch per step leaves in them. */
 int lbm_variant_info(int variant, int* block, int* cells_per_thread, int* vec, int* flags);
 int lbm_set_variant(lbm_handle* h, int variant);
 int lbm_get_variant(lbm_handle* h, int* variant);

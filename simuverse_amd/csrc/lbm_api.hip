@@ -85,6 +85,7 @@ struct lbm_handle {
     float omega = 1.0f;
     float scale = 1.0f, inv_scale = 1.0f;
     int variant = 6;
+    bool auto_shape = true;  // no shape chosen by the caller: lbm_run takes default_shape's
     int graph_chunk = 100;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -175,15 +176,35 @@ hipError_t enqueue_step(lbm_handle* h, int swap, bool export_macro)
 
 // Steps one launch advances: 2 or 3 for a multi-step variant on a plain
 // physics handle, else 1.
-int launch_steps(const lbm_handle* h) { return h->physics() && !h->mlp ? step_variant_steps(h->variant) : 1; }
+// The shape lbm_run steps with: the caller's (lbm_set_variant, lbm_autotune),
+// else the one the lattice's size asks for.
+int run_variant(const lbm_handle* h)
+{
+    return h->auto_shape ? default_step_variant(h->f16, h->d.nx, h->d.ny, h->d.x_edge, h->variant) : h->variant;
+}
+
+int launch_steps(const lbm_handle* h) { return h->physics() && !h->mlp ? step_variant_steps(run_variant(h)) : 1; }
+
+// Steps at the end of a run that take one-step launches whatever is left
+// over: without a shape chosen by the caller the other buffer holds the
+// state one step before the current one after every run, as it does when
+// every step is a launch of its own.
+int single_tail(const lbm_handle* h, bool export_macro)
+{
+    return h->auto_shape && launch_steps(h) > 1 && !export_macro ? 1 : 0;
+}
 
 // launch_steps(h) steps from buffer `swap` into buffer 1-swap in one launch.
 hipError_t enqueue_multi(lbm_handle* h, int swap)
 {
-    if (launch_steps(h) == 3)
-        return launch_phys_step3(h->variant, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[swap],
+    const int v = run_variant(h);
+    if (kStepVariants[v].flags & kNStep)
+        return launch_phys_stepn(v, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[swap],
                                  h->buf[swap ^ 1], h->bits, h->words, h->stream);
-    return launch_phys_step2(h->variant, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[swap],
+    if (launch_steps(h) == 3)
+        return launch_phys_step3(v, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[swap],
+                                 h->buf[swap ^ 1], h->bits, h->words, h->stream);
+    return launch_phys_step2(v, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[swap],
                              h->buf[swap ^ 1], h->bits, h->words, h->stream);
 }
 
@@ -232,7 +253,8 @@ int ensure_graph(lbm_handle* h, int b)
 // Enqueue nsteps steps from the current buffer (no synchronisation).
 int enqueue_run(lbm_handle* h, int nsteps, bool export_macro)
 {
-    int plain = export_macro ? nsteps - 1 : nsteps;
+    const int tail = nsteps > 0 ? single_tail(h, export_macro) : 0;
+    int plain = (export_macro ? nsteps - 1 : nsteps) - tail;
     if (h->graph_chunk > 0) {
         while (plain >= h->graph_chunk) {
             int rc = ensure_graph(h, h->cur);
@@ -249,7 +271,7 @@ int enqueue_run(lbm_handle* h, int nsteps, bool export_macro)
             h->cur ^= 1;
         }
     }
-    for (int s = 0; s < plain; ++s) {
+    for (int s = 0; s < plain + tail; ++s) {
         HIP_TRY(enqueue_step(h, h->cur, false));
         h->cur ^= 1;
     }
@@ -764,8 +786,9 @@ int lbm_set_variant(lbm_handle* h, int variant)
         return fail(LBM_ERR_INVALID, "variant %d does not fit a %dx%d lattice with x edge %d (see lbm_variant_info)",
                     variant, h->d.nx, h->d.ny, h->d.x_edge);
     HIP_TRY(hipStreamSynchronize(h->stream));
-    if (variant != h->variant) drop_graphs(h);
+    if (variant != h->variant || h->auto_shape) drop_graphs(h);
     h->variant = variant;
+    h->auto_shape = false;
     return LBM_OK;
 }
 
@@ -809,7 +832,10 @@ int lbm_autotune(lbm_handle* h, int steps, int* best_variant, double* ms_per_ste
         if (!step_variant_ok(v, h->d.nx, h->d.ny, h->d.x_edge)) continue;
         const int per = step_variant_steps(v);  // steps per launch
         auto launch = [&]() {
-            hipError_t r = per == 3   ? launch_phys_step3(v, h->f16, h->d.x_edge, h->force(), h->phys(),
+            hipError_t r = (kStepVariants[v].flags & kNStep)
+                               ? launch_phys_stepn(v, h->f16, h->d.x_edge, h->force(), h->phys(), h->buf[h->cur],
+                                                   h->buf[h->cur ^ 1], h->bits, h->words, h->stream)
+                           : per == 3   ? launch_phys_step3(v, h->f16, h->d.x_edge, h->force(), h->phys(),
                                                           h->buf[h->cur], h->buf[h->cur ^ 1], h->bits, h->words,
                                                           h->stream)
                            : per == 2 ? launch_phys_step2(v, h->f16, h->d.x_edge, h->force(), h->phys(),
@@ -839,8 +865,9 @@ int lbm_autotune(lbm_handle* h, int steps, int* best_variant, double* ms_per_ste
     (void)hipFree(saved);
     h->cur = cur0;
     if (e != hipSuccess) return fail(LBM_ERR_HIP, "autotune: %s", hipGetErrorString(e));
-    if (best != h->variant) drop_graphs(h);
+    if (best != h->variant || h->auto_shape) drop_graphs(h);
     h->variant = best;
+    h->auto_shape = false;
     if (best_variant) *best_variant = best;
     if (ms_per_step) *ms_per_step = best_ms;
     return LBM_OK;

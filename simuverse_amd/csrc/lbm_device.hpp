@@ -89,8 +89,12 @@ enum : int {
     kTwoStep = 16, // two steps per launch through an LDS tile (temporal blocking)
     kGridStride = 32, // batched: block b takes chunks b, b + grid, ... (else a contiguous range)
     kThreeStep = 64,  // three steps per launch through an LDS tile with a two-cell ring
-    kRowStream = 128  // two-step: strips of block-size columns streamed down a chunk of rows
+    kRowStream = 128, // two-step: strips of block-size columns streamed down a chunk of rows
+    kNStep = 256      // several steps per launch, their number in bits kNStepShift.. (k_phys_stepn)
 };
+
+constexpr int kNStepShift = 12;
+constexpr int n_step_flags(int ns) { return kNStep | (ns << kNStepShift); }
 
 // Population storage of the physics mode.  Kernels work on deviations
 // g_i = f_i - w_i from the rest state, and memory holds the deviation too, so

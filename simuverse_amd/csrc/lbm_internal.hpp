@@ -16,12 +16,13 @@ struct StepVariant {
     int block;             // threads per block
     int cells_per_thread;  // cells handled by one thread
     int vec;               // consecutive cells per lane (1: strided by block)
-    int flags;             // kNtStore | kNtLoad | kXcdRemap | kShfl | kTwoStep | kThreeStep | kRowStream
+    int flags;             // kNtStore | kNtLoad | kXcdRemap | kShfl | kTwoStep | kThreeStep | kRowStream | kNStep
 };
 // kTwoStep and kThreeStep variants: cells_per_thread = tile (or chunk)
 // rows, vec = tile (or strip) width; one launch advances two steps
 // (launch_phys_step2) or three (launch_phys_step3), and the steps left over
-// use the one-step variant kSingleStepFallback.
+// use the one-step variant kSingleStepFallback.  kNStep variants likewise,
+// with the number of steps in the flags (launch_phys_stepn).
 constexpr int kSingleStepFallback = 6;
 // The autotuners keep the fastest shape, but a later shape in the table
 // replaces the best so far only when it is at least 1 % faster: shapes of
@@ -32,15 +33,25 @@ constexpr double kTuneMargin = 0.99;
 extern const StepVariant kStepVariants[];
 extern const int kNumStepVariants;
 bool step_variant_ok(int variant, int nx, int ny, int xedge);
+// The shape for a lattice whose caller chose none: an N-step shape by the
+// lattice's size, or `one_step` where none fits.
+int default_step_variant(bool f16, int nx, int ny, int xedge, int one_step);
 inline bool step_variant_two_step(int variant) { return (kStepVariants[variant].flags & kTwoStep) != 0; }
-// Steps one launch of a variant advances: 1, 2 (kTwoStep) or 3 (kThreeStep).
+// Steps one launch of a variant advances: 1, 2 (kTwoStep), 3 (kThreeStep) or the flags' number (kNStep).
 inline int step_variant_steps(int variant)
 {
     const int f = kStepVariants[variant].flags;
+    if (f & kNStep) return f >> kNStepShift;
     return (f & kThreeStep) ? 3 : ((f & kTwoStep) ? 2 : 1);
 }
 // Whether two-step tiles of width bw fit an nx x ny lattice (lbm_step2.hip).
 bool two_step_fits(int bw, int nx, int ny, int xedge);
+// Whether ns-step tiles of width bw fit (lbm_stepn.hip): the two-step rule,
+// and a ring of ns - 1 cells that wraps around the lattice at most once.
+inline bool nstep_fits(int bw, int ns, int nx, int ny, int xedge)
+{
+    return nx >= ns && ny >= ns && two_step_fits(bw, nx, ny, xedge);
+}
 // Blocks of bs threads for n work items.
 inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -54,6 +65,8 @@ hipError_t launch_phys_step(int variant, bool f16, int xedge, bool force, bool e
 hipError_t launch_phys_step2(int variant, bool f16, int xedge, bool force, const PhysArgs& a, const void* src,
                              void* dst, const uint32_t* bits, uint32_t words, hipStream_t s);
 hipError_t launch_phys_step3(int variant, bool f16, int xedge, bool force, const PhysArgs& a, const void* src,
+                             void* dst, const uint32_t* bits, uint32_t words, hipStream_t s);
+hipError_t launch_phys_stepn(int variant, bool f16, int xedge, bool force, const PhysArgs& a, const void* src,
                              void* dst, const uint32_t* bits, uint32_t words, hipStream_t s);
 hipError_t launch_phys_macro(bool f16, int xedge, bool force, const PhysArgs& a, const void* src,
                              const uint8_t* mat, float* rho, float* ux, float* uy, hipStream_t s);

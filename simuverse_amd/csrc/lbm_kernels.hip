@@ -793,6 +793,11 @@ const StepVariant kStepVariants[] = {
     {256, 8, 64, kNtStore | kThreeStep},
     {768, 24, 64, kNtStore | kThreeStep | kXcdRemap},
     {768, 24, 64, kNtStore | kThreeStep},
+    // N steps per launch, each thread bound to its cells: (block, tile rows, tile width, flags)
+    {1024, 16, 16, n_step_flags(9)},
+    {1024, 24, 24, kXcdRemap | n_step_flags(5)},
+    {1024, 24, 56, kXcdRemap | n_step_flags(5)},
+    {1024, 40, 56, kXcdRemap | n_step_flags(5)},
 };
 const int kNumStepVariants = (int)(sizeof(kStepVariants) / sizeof(kStepVariants[0]));
 
@@ -800,9 +805,40 @@ bool step_variant_ok(int v, int nx, int ny, int xedge)
 {
     if (v < 0 || v >= kNumStepVariants) return false;
     const StepVariant& sv = kStepVariants[v];
+    if (sv.flags & kNStep) return nstep_fits(sv.vec, sv.flags >> kNStepShift, nx, ny, xedge);
     if (sv.flags & (kTwoStep | kThreeStep)) return two_step_fits(sv.vec, nx, ny, xedge);
     if (sv.flags & kShfl) return xedge == 0 && nx % (sv.block * sv.vec) == 0;
     return sv.vec == 1 || nx % sv.vec == 0;
+}
+
+// Microseconds per step, channel without force in binary32 (one-step shape,
+// 48: 16 x 16 tiles and nine steps, 49: 24 x 24 and five, 50: 56 x 24 and
+// five; binary16 and periodic lattices order the same way):
+//            one-step   48     49     50
+//   128x100     3.24   1.18   1.47   2.42
+//   256x256     3.75   1.29   1.51   2.40   256 tiles of 48: one per CU
+//   350x300     4.47   1.77   1.57   2.43
+//   1024x1024   15.4   9.05   5.40   5.72   1849 tiles of 49
+//   1531x1037   21.4   13.1   7.80   7.10   2816
+//   8192x8192   755    481    292    226
+// One block per CU hides nothing, so while one round of blocks covers the
+// lattice the launches count and the deepest shape wins; then the smaller
+// block, of which more fit the tail of the last round; then the least ring:
+// in binary16, where two blocks of it share a CU, 51 (56 x 40 and five;
+// 8192x8192 with force 253 against 279 for 50; in binary32 371 against 273).
+int default_step_variant(bool f16, int nx, int ny, int xedge, int one_step)
+{
+    constexpr int64_t kCus = 256;
+    const auto tiles = [&](int v) {
+        const int64_t bw = kStepVariants[v].vec, bh = kStepVariants[v].cells_per_thread;
+        return ((nx + bw - 1) / bw) * ((ny + bh - 1) / bh);
+    };
+    if (tiles(48) <= kCus && step_variant_ok(48, nx, ny, xedge)) return 48;
+    if (tiles(49) <= 8 * kCus && step_variant_ok(49, nx, ny, xedge)) return 49;
+    if (f16 && step_variant_ok(51, nx, ny, xedge)) return 51;
+    for (int v : {50, 49, 48})
+        if (step_variant_ok(v, nx, ny, xedge)) return v;
+    return one_step;
 }
 
 template <typename T, int XEDGE, bool FORCE, bool EXPORT>

@@ -236,7 +236,9 @@ def variant_shapes() -> list[tuple[int, int, int, int]]:
     steps per launch through an LDS tile of cells_per_thread rows x vec
     cells, 64 three steps per launch through an LDS tile of cells_per_thread
     rows x vec cells with a two-cell ring, 128 the two steps streamed down
-    strips of vec columns in chunks of cells_per_thread rows)."""
+    strips of vec columns in chunks of cells_per_thread rows, 256 flags >> 12
+    steps per launch through an LDS tile of cells_per_thread rows x vec
+    cells)."""
     lib = load_library()
     out = []
     for v in range(lib.lbm_variant_count()):
@@ -248,15 +250,15 @@ def variant_shapes() -> list[tuple[int, int, int, int]]:
 
 def variant_ok(variant: int, nx: int, ny: int, x_edge: int = X_PERIODIC) -> bool:
     """Whether a tile variant can step an nx x ny lattice (the library's
-    own rule: two- and three-step variants need nx, ny >= 3, with the
-    inlet/outlet edge a last tile of at least two columns (nx % vec != 1),
+    own rule: multi-step variants need nx, ny >= 3, and at least the number
+    of steps where the flags hold it, with the inlet/outlet edge a last tile of at least two columns (nx % vec != 1),
     and rows and row stride below 2^24 (ny < 2^24, 9 (nx + 16) < 2^24);
     lane-shuffle variants need periodic x and whole blocks of block*vec
     cells per row; vector variants need nx % vec == 0)."""
     b, c, v, f = variant_shapes()[variant]
-    if f & (16 | 64):
-        return (nx >= 3 and ny >= 3 and (x_edge == X_PERIODIC or nx % v != 1) and 9 * (nx + 16) < (1 << 24)
-                and ny < (1 << 24))
+    if f & (16 | 64 | 256):
+        return (min(nx, ny) >= (f >> 12 if f & 256 else 3) and (x_edge == X_PERIODIC or nx % v != 1)
+                and 9 * (nx + 16) < (1 << 24) and ny < (1 << 24))
     if f & 8:
         return x_edge == X_PERIODIC and nx % (b * v) == 0
     return v == 1 or nx % v == 0
