@@ -335,7 +335,7 @@ def run_batch(args):
     bpc = 36 if args.f16 else 72
     variant = b.variant()
     block, vec, tile_h, flags = L.batch_variant_shapes()[variant]
-    per_launch = 3 if flags & 64 else (2 if flags & 16 else 1)
+    per_launch = flags >> 12 if flags & 256 else (3 if flags & 64 else (2 if flags & 16 else 1))
     workload = f"d2q9_batch512_{'f16dev' if args.f16 else 'f32'}"
     roof = roofline(bpc, cells, step_s, per_launch, traffic_from_profiles(workload, variant))
     # Domains whose state is no longer finite (BGK at tau near 1/2 with a
@@ -362,7 +362,8 @@ def run_batch(args):
         "dtype": "f16-deviation storage, f32 math" if args.f16 else "f32",
         "data": "synthetic",
         "config": {"workload": workload, "domains": len(doms), "cells": int(cells), "variant": variant,
-                   "batch_variant": {"kernel": {3: "k_batch_step3", 2: "k_batch_step2"}.get(per_launch, "k_batch_step"),
+                   "batch_variant": {"kernel": "k_batch_stepn" if flags & 256 else
+                                     {3: "k_batch_step3", 2: "k_batch_step2"}.get(per_launch, "k_batch_step"),
                                      "block": block, "vec": vec, "tile_rows": tile_h, "flags": flags},
                    "graph_chunk": args.graph_chunk, "seed": W.SEED,
                    "finite_domains": len(doms) - len(diverged), "diverged_domains": diverged,

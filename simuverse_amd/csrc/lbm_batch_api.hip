@@ -47,7 +47,7 @@ struct lbm_batch {
     BatchDomainDev* ddom = nullptr;
     uint16_t* chunk_dom = nullptr;  // chunk -> domain for the one-step variant in use
     uint32_t nchunks = 0;
-    uint16_t* tile_dom = nullptr;   // tile -> domain for a two- or three-step variant
+    uint16_t* tile_dom = nullptr;   // tile -> domain for a multi-step variant
     uint32_t ntiles = 0;
     float* tmp3 = nullptr;
     double* partial = nullptr;
@@ -61,7 +61,7 @@ struct lbm_batch {
 
     PhysArgs args(int d) const { return dom[d].a; }
     void* view(int b, int d) const { return (char*)buf[b] + (size_t)dom[d].pop_off * elem; }
-    // steps one launch of the chosen variant advances (1, 2 or 3)
+    // steps one launch of the chosen variant advances
     int steps() const { return batch_variant_steps(variant); }
     // the variant of single steps: the chosen one, or the fallback of a multi-step one
     int step1_variant() const { return steps() > 1 ? kBatchSingleStepFallback : variant; }
@@ -120,7 +120,7 @@ int upload_table(lbm_batch* b, const std::vector<uint16_t>& table, uint16_t** de
 
 // Work tables of the current variant: chunks of block*vec cells for the
 // one-step variant (the chosen one or the multi-step fallback), and tiles
-// for a two- or three-step variant.
+// for a multi-step variant.
 int build_chunks(lbm_batch* b)
 {
     const BatchVariant& sv = kBatchVariants[b->step1_variant()];
@@ -154,7 +154,9 @@ bool batch_variant_ok(const lbm_batch* b, int v)
     if (v < 0 || v >= kNumBatchVariants) return false;
     if (batch_variant_steps(v) == 1) return true;
     for (const lbm_domain_desc& q : b->desc)
-        if (!two_step_fits(kBatchVariants[v].vec, q.nx, q.ny, q.x_edge != LBM_X_PERIODIC ? 1 : 0)) return false;
+        if (!nstep_fits(kBatchVariants[v].vec, std::max(3, batch_variant_steps(v)), q.nx, q.ny,
+                        q.x_edge != LBM_X_PERIODIC ? 1 : 0))
+            return false;
     return true;
 }
 
@@ -168,6 +170,9 @@ hipError_t batch_enqueue_step(lbm_batch* b, int swap)
 // b->steps() steps from buffer `swap` into buffer 1-swap (multi-step variant).
 hipError_t batch_enqueue_multi(lbm_batch* b, int swap)
 {
+    if (kBatchVariants[b->variant].flags & kNStep)
+        return launch_batch_stepn(b->variant, b->f16, b->ddom, b->tile_dom, b->ntiles, b->buf[swap], b->buf[swap ^ 1],
+                                  b->bits, b->stream);
     if (b->steps() == 3)
         return launch_batch_step3(b->variant, b->f16, b->ddom, b->tile_dom, b->ntiles, b->buf[swap],
                                   b->buf[swap ^ 1], b->bits, b->stream);

@@ -101,19 +101,20 @@ hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t s
 // counts take the one-step variant kBatchSingleStepFallback.
 struct BatchVariant {
     int block;           // threads per block
-    int vec;             // consecutive cells per lane; tile width when two- or three-step
+    int vec;             // consecutive cells per lane; tile width when multi-step
     int blocks_per_cu;   // persistent grid = blocks_per_cu * CUs (one-step)
-    int flags;           // kNtStore | kXcdRemap | kGridStride | kTwoStep | kThreeStep
-    int tile_h;          // tile rows (two- and three-step)
+    int flags;           // kNtStore | kXcdRemap | kGridStride | kTwoStep | kThreeStep | kNStep
+    int tile_h;          // tile rows (multi-step)
 };
 constexpr int kBatchSingleStepFallback = 9;
 extern const BatchVariant kBatchVariants[];
 extern const int kNumBatchVariants;
 inline bool batch_variant_two_step(int variant) { return (kBatchVariants[variant].flags & kTwoStep) != 0; }
-// Steps one launch of a batch variant advances: 1, 2 (kTwoStep) or 3 (kThreeStep).
+// Steps one launch of a batch variant advances: 1, 2 (kTwoStep), 3 (kThreeStep) or the flags' number (kNStep).
 inline int batch_variant_steps(int variant)
 {
     const int f = kBatchVariants[variant].flags;
+    if (f & kNStep) return f >> kNStepShift;
     return (f & kThreeStep) ? 3 : ((f & kTwoStep) ? 2 : 1);
 }
 hipError_t launch_batch_step(int variant, bool f16, const BatchDomainDev* doms, const uint16_t* chunk_dom,
@@ -125,6 +126,9 @@ hipError_t launch_batch_step2(int variant, bool f16, const BatchDomainDev* doms,
                               uint32_t ntiles, const void* src, void* dst, const uint32_t* bits, hipStream_t s);
 // Three steps of every domain, with the tiles of a three-step variant.
 hipError_t launch_batch_step3(int variant, bool f16, const BatchDomainDev* doms, const uint16_t* tile_dom,
+                              uint32_t ntiles, const void* src, void* dst, const uint32_t* bits, hipStream_t s);
+// Several steps of every domain, with the tiles of an N-step variant.
+hipError_t launch_batch_stepn(int variant, bool f16, const BatchDomainDev* doms, const uint16_t* tile_dom,
                               uint32_t ntiles, const void* src, void* dst, const uint32_t* bits, hipStream_t s);
 
 // Learned collision, restriction and health check.

@@ -525,6 +525,9 @@ const BatchVariant kBatchVariants[] = {
     {256, 64, 0, kNtStore | kThreeStep, 8},
     {768, 64, 0, kNtStore | kThreeStep, 24}, {768, 64, 0, kNtStore | kThreeStep | kXcdRemap, 24},
     {1024, 64, 0, kNtStore | kThreeStep, 32},
+    // N steps per launch (launch_batch_stepn): (block, tile width, -, flags, tile rows)
+    {1024, 24, 0, kXcdRemap | n_step_flags(5), 24}, {1024, 56, 0, kXcdRemap | n_step_flags(5), 24},
+    {1024, 56, 0, kXcdRemap | n_step_flags(5), 40},
 };
 const int kNumBatchVariants = (int)(sizeof(kBatchVariants) / sizeof(kBatchVariants[0]));
 

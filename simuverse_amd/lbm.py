@@ -772,7 +772,7 @@ def batch_variant_shapes() -> list[tuple[int, int, int, int]]:
     width, multi-step tile rows (0 for one-step variants), flags: 1
     non-temporal stores, 4 work grouped per XCD, 16 two steps per launch,
     32 persistent blocks take every grid-th chunk, 64 three steps per
-    launch)."""
+    launch, 256 flags >> 12 steps per launch)."""
     lib = load_library()
     out = []
     for v in range(lib.lbm_batch_variant_count()):
