@@ -26,6 +26,7 @@
 #include "lbm3d.h"
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
+#include "lbm_readback.hpp"
 
 namespace lbm {
 namespace d3 {
@@ -469,6 +470,7 @@ struct lbm3d_handle {
     int graph_chunk = 100;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    Staging staging;  // of the readbacks
 };
 
 namespace {
@@ -720,8 +722,8 @@ int lbm3d_read_populations(lbm3d_handle* h, float* f)
         hipLaunchKernelGGL((k3_dev_to_host<float>), dim3(blocks256(h->cells)), dim3(256), 0, h->stream, h->a,
                            (const float*)h->buf[h->cur], stage);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(f, stage, bytes, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    const HostPiece p{f, stage, bytes};
+    if (e == hipSuccess) e = h->staging.to_host(&p, 1, h->stream, h->dev);
     (void)hipFree(stage);
     if (e != hipSuccess) return lbm_fail(LBM_ERR_HIP, "3-D population download: %s", hipGetErrorString(e));
     return LBM_OK;
@@ -771,11 +773,9 @@ int lbm3d_macro(lbm3d_handle* h, float* rho, float* ux, float* uy, float* uz)
                            (const float*)h->buf[h->cur], h->mat, h->macro);
     TRY3(hipGetLastError());
     float* dsts[4] = {rho, ux, uy, uz};
-    for (int k = 0; k < 4; ++k)
-        if (dsts[k])
-            TRY3(hipMemcpyAsync(dsts[k], h->macro + (size_t)k * h->cells, h->cells * sizeof(float),
-                                hipMemcpyDeviceToHost, h->stream));
-    TRY3(hipStreamSynchronize(h->stream));
+    HostPiece p[4];
+    for (int k = 0; k < 4; ++k) p[k] = {dsts[k], h->macro + (size_t)k * h->cells, h->cells * sizeof(float)};
+    TRY3(h->staging.to_host(p, 4, h->stream, h->dev));
     return LBM_OK;
 }
 

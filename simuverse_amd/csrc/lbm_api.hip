@@ -16,6 +16,7 @@
 
 #include "lbm.h"
 #include "lbm_internal.hpp"
+#include "lbm_readback.hpp"
 
 using namespace lbm;
 
@@ -94,6 +95,7 @@ struct lbm_handle {
     int mlp_precision = LBM_MLP_BF16;
     uint32_t* health = nullptr;     // [max |u|^2 bits, non-finite flag]
     void* backup = nullptr;         // chunk start state of lbm_run_guarded
+    Staging staging;                // of the readbacks
 
     bool physics() const { return d.mode == LBM_MODE_PHYSICS; }
     bool force() const { return d.force_x != 0.0f || d.force_y != 0.0f; }
@@ -497,6 +499,8 @@ int lbm_create(const lbm_desc* desc, lbm_handle** out)
         free_handle(h);
         return fail(LBM_ERR_HIP, "stream/event setup: %s", hipGetErrorString(e));
     }
+    // a frame's readback finds its slots ready; larger ones add theirs when they come
+    (void)h->staging.reserve(std::min<size_t>(12 * n, 2u << 20));
     rc = do_reset(h);
     if (rc != LBM_OK) {
         std::string msg = g_last_error;
@@ -613,8 +617,8 @@ int lbm_read_populations(lbm_handle* h, int buf, float* f)
         float* stage = nullptr;
         HIP_TRY(hipMalloc(&stage, 9 * nb));
         hipError_t e = launch_dev_to_host(h->f16, h->phys(), h->buf[buf], stage, h->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(f, stage, 9 * nb, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        const HostPiece p{f, stage, 9 * nb};
+        if (e == hipSuccess) e = h->staging.to_host(&p, 1, h->stream, h->dev);
         (void)hipFree(stage);
         if (e != hipSuccess) return fail(LBM_ERR_HIP, "population download: %s", hipGetErrorString(e));
     }
@@ -688,10 +692,8 @@ int lbm_read_macro(lbm_handle* h, float* rho, float* ux, float* uy)
     int rc = check_handle(h);
     if (rc) return rc;
     const size_t nb = (size_t)h->n * sizeof(float);
-    if (ux) HIP_TRY(hipMemcpyAsync(ux, h->macro, nb, hipMemcpyDeviceToHost, h->stream));
-    if (uy) HIP_TRY(hipMemcpyAsync(uy, h->macro + h->n, nb, hipMemcpyDeviceToHost, h->stream));
-    if (rho) HIP_TRY(hipMemcpyAsync(rho, h->macro + 2 * (size_t)h->n, nb, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    const HostPiece p[3] = {{ux, h->macro, nb}, {uy, h->macro + h->n, nb}, {rho, h->macro + 2 * (size_t)h->n, nb}};
+    HIP_TRY(h->staging.to_host(p, 3, h->stream, h->dev));
     return LBM_OK;
 }
 
@@ -710,8 +712,8 @@ int lbm_read_macro_rgba16f(lbm_handle* h, uint16_t* rgba)
     if (!rgba) return fail(LBM_ERR_INVALID, "null output");
     if ((rc = ensure_texels(h))) return rc;
     HIP_TRY(launch_pack_rgba16f(h->macro, h->n, h->texels, h->stream));
-    HIP_TRY(hipMemcpyAsync(rgba, h->texels, (size_t)h->n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    const HostPiece p{rgba, h->texels, (size_t)h->n * 8};
+    HIP_TRY(h->staging.to_host(&p, 1, h->stream, h->dev));
     return LBM_OK;
 }
 
@@ -722,8 +724,8 @@ int lbm_read_curl_rgba16f(lbm_handle* h, uint16_t* rgba)
     if (!rgba) return fail(LBM_ERR_INVALID, "null output");
     if ((rc = ensure_texels(h))) return rc;
     HIP_TRY(launch_curl_rgba16f(h->macro, h->d.nx, h->d.ny, h->texels, h->stream));
-    HIP_TRY(hipMemcpyAsync(rgba, h->texels, (size_t)h->n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    const HostPiece p{rgba, h->texels, (size_t)h->n * 8};
+    HIP_TRY(h->staging.to_host(&p, 1, h->stream, h->dev));
     return LBM_OK;
 }
 
@@ -740,10 +742,8 @@ int lbm_macro(lbm_handle* h, float* rho, float* ux, float* uy)
     else
         HIP_TRY(launch_wgsl_macro(h->wgsl(), (const float*)h->buf[h->cur], h->mat, h->fvel, r, u, v, h->stream));
     const size_t nb = (size_t)h->n * sizeof(float);
-    if (rho) HIP_TRY(hipMemcpyAsync(rho, r, nb, hipMemcpyDeviceToHost, h->stream));
-    if (ux) HIP_TRY(hipMemcpyAsync(ux, u, nb, hipMemcpyDeviceToHost, h->stream));
-    if (uy) HIP_TRY(hipMemcpyAsync(uy, v, nb, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    const HostPiece p[3] = {{rho, r, nb}, {ux, u, nb}, {uy, v, nb}};
+    HIP_TRY(h->staging.to_host(p, 3, h->stream, h->dev));
     return LBM_OK;
 }
 
@@ -888,9 +888,8 @@ int lbm_save_state(lbm_handle* h, void* out, size_t bytes)
         return fail(LBM_ERR_INVALID, "state buffer must be %zu bytes", sizeof(StateHeader) + h->pop_bytes());
     const StateHeader hd = state_header(h);
     std::memcpy(out, &hd, sizeof hd);
-    HIP_TRY(hipMemcpyAsync(static_cast<char*>(out) + sizeof hd, h->buf[h->cur], h->pop_bytes(),
-                           hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    const HostPiece p{static_cast<char*>(out) + sizeof hd, h->buf[h->cur], h->pop_bytes()};
+    HIP_TRY(h->staging.to_host(&p, 1, h->stream, h->dev));
     return LBM_OK;
 }
 

@@ -19,6 +19,7 @@
 
 #include "lbm.h"
 #include "lbm_internal.hpp"
+#include "lbm_readback.hpp"
 
 using namespace lbm;
 
@@ -58,6 +59,7 @@ struct lbm_batch {
     int graph_chunk = 100;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    Staging staging;  // of the readbacks
 
     PhysArgs args(int d) const { return dom[d].a; }
     void* view(int b, int d) const { return (char*)buf[b] + (size_t)dom[d].pop_off * elem; }
@@ -448,8 +450,8 @@ int lbm_batch_read_populations(lbm_batch* b, int d, float* f)
     float* stage = nullptr;
     BATCH_TRY(hipMalloc(&stage, 9 * nb));
     hipError_t e = launch_dev_to_host(b->f16, b->dom[d].a, b->view(b->cur, d), stage, b->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(f, stage, 9 * nb, hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+    const HostPiece p{f, stage, 9 * nb};
+    if (e == hipSuccess) e = b->staging.to_host(&p, 1, b->stream, b->dev);
     (void)hipFree(stage);
     if (e != hipSuccess) return lbm_fail(LBM_ERR_HIP, "population download: %s", hipGetErrorString(e));
     return LBM_OK;
@@ -497,10 +499,11 @@ int lbm_batch_macro(lbm_batch* b, int d, float* rho, float* ux, float* uy)
     float* v = u + n;
     BATCH_TRY(launch_phys_macro(b->f16, b->dom[d].x_edge, b->dom[d].force != 0, b->args(d), b->view(b->cur, d),
                                 b->mat + b->cell_off[d], r, u, v, b->stream));
-    if (rho) BATCH_TRY(hipMemcpyAsync(rho, r, n * sizeof(float), hipMemcpyDeviceToHost, b->stream));
-    if (ux) BATCH_TRY(hipMemcpyAsync(ux, u, n * sizeof(float), hipMemcpyDeviceToHost, b->stream));
-    if (uy) BATCH_TRY(hipMemcpyAsync(uy, v, n * sizeof(float), hipMemcpyDeviceToHost, b->stream));
-    BATCH_TRY(hipStreamSynchronize(b->stream));
+    // room for the largest domain at once: a program reads them one after the other
+    (void)b->staging.reserve((size_t)3 * b->max_cells * sizeof(float));
+    const size_t nb = n * sizeof(float);
+    const HostPiece p[3] = {{rho, r, nb}, {ux, u, nb}, {uy, v, nb}};
+    BATCH_TRY(b->staging.to_host(p, 3, b->stream, b->dev));
     return LBM_OK;
 }
 
