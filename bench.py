@@ -408,7 +408,8 @@ def run_d3q19(args):
     step_s = ms / 1e3 / K
     bpc = 76 if args.f16 else 152
     workload = f"d3q19_{'f16dev' if args.f16 else 'f32'}_{n}cubed"
-    roof = roofline(bpc, cells, step_s, 1, traffic_from_profiles(workload, variant))
+    block, cpt, flags = L.variant3_shapes()[variant]
+    roof = roofline(bpc, cells, step_s, 2 if flags & 16 else 1, traffic_from_profiles(workload, variant))
     r = lat.reduce()
     log(f"{K} steps: {ms:.1f} ms, {step_s * 1e6:.2f} us/step, {cells / step_s / 1e6:.0f} MLUPS, {roof['achieved']:.0f} GB/s; "
         f"mass {r[0]:.9e} drag ({r[4]:.3e}, {r[5]:.3e}, {r[6]:.3e})")
@@ -419,7 +420,6 @@ def run_d3q19(args):
         # the numpy oracle takes about 5 s per step at 256^3
         acc = accuracy_d3q19(lat, scene, tau, (g, 0.0, 0.0), min(args.accuracy_steps, 5))
         log(f"d3q19 accuracy vs binary64 oracle: {acc}")
-    block, cpt, flags = L.variant3_shapes()[variant]
     line = {
         "metric": METRIC,
         "value": round(cells / step_s / 1e6, 1),
@@ -436,7 +436,7 @@ def run_d3q19(args):
         "config": {"workload": workload, "nx": n, "ny": n, "nz": n, "tau": tau, "body_force": [g, 0.0, 0.0],
                    "solid_fraction": round(scene.solid_fraction, 5), "spheres": int(len(scene.spheres)),
                    "seed": W.SEED, "variant": variant,
-                   "tile_variant": {"kernel": "k3_step", "block": block, "cells_per_thread": cpt, "flags": flags},
+                   "tile_variant": {"kernel": "k3_step2" if flags & 16 else "k3_step", "block": block, "cells_per_thread": cpt, "flags": flags},
                    "graph_chunk": args.graph_chunk},
         "roofline": roof,
         "accuracy": acc,

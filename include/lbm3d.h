@@ -77,7 +77,12 @@ int lbm3d_reduce(lbm3d_handle* h, double out[7]);
 int lbm3d_variant_count(void);
 /* block: threads per block; cells_per_thread: cells of one row per thread
  * (strided by the block); flags: bit 0 non-temporal population stores,
- * bit 2 the blocks one XCD receives take a contiguous range of rows. */
+ * bit 2 the blocks one XCD receives take a contiguous range of rows, bit 4
+ * two steps per launch, streamed along z, with cells_per_thread the width of
+ * a block's region (one slab must lie under 4 GiB; launches go in pairs, the
+ * steps left over run one per launch).  Until a shape is chosen, lbm3d_run
+ * takes 256 threads with plain stores where both buffers fit the 256 MB
+ * cache and with non-temporal ones beyond. */
 int lbm3d_variant_info(int variant, int* block, int* cells_per_thread, int* flags);
 int lbm3d_set_variant(lbm3d_handle* h, int variant);
 int lbm3d_get_variant(lbm3d_handle* h, int* variant);

@@ -126,7 +126,9 @@ __device__ inline void collide3(const Args3& a, float g[19], float rho, float ux
         const float q = fmaf(eu, fmaf(4.5f, eu, 3.0f), -usq);
         const float geq = fmaf(wr[k], q, wd[k]);
         float out = fmaf(-a.omega, g[i] - geq, g[i]);
-        if (FORCE) out += fmaf(a.fb[i], eu, fmaf(-a.fc[k], ug, a.fa[i]));
+        // fa and fb flip sign with the direction: the odd ones of each pair serve both
+        if (FORCE && (i == 0 || (i & 1))) out += fmaf(a.fb[i], eu, fmaf(-a.fc[k], ug, a.fa[i]));
+        else if (FORCE) out += fmaf(-a.fb[i - 1], eu, fmaf(-a.fc[k], ug, -a.fa[i - 1]));
         g[i] = out;
     }
 }
@@ -222,6 +224,180 @@ __global__ __launch_bounds__(BS) void k3_step(Args3 a, const T* __restrict__ src
     for (int k = 0; k < CPT; ++k) {
         const int x = x0 + k * BS;
         if (x < a.nx) cell3<T, FORCE, FLAGS>(a, src, dst, bits, words, x, y, z);
+    }
+}
+
+// Two steps per launch, streamed along z.  A block of BS threads owns a region
+// of RW x (BS / RW) columns, one per thread: a tile with a ring of one cell,
+// and a chunk of `depth` slabs.  It walks up the chunk; each turn computes
+// step 1 of slab z + 1 (gathered from memory as the one-step kernel does),
+// puts the populations that move sideways into LDS, and then computes step 2
+// of slab z from there.  LDS holds what a step 2 can pull: the four that move
+// up of slabs z - 1 .. z + 1, the eight that stay level and the four that move
+// down of z and z + 1 (36 values a column); the rest population and the two
+// that move straight up and down stay in the thread's registers.  A
+// population from a solid cell is the thread's own opposite one of slab z,
+// which is in the same places.  Step 1 rounds to the storage type as a launch
+// of its own would, so the destination is what two one-step launches leave,
+// bit for bit at every slot a fluid cell can read.
+//
+// The one-step kernel is bound by HBM (152 B per cell and step in binary32);
+// here two steps share one read, with the ring's, and one write, and what
+// bounds it is each turn's chain (loads a turn ahead, collision, barrier,
+// pulls, collision, stores) with 16 wavefronts on a CU.  The autotuner takes
+// it in binary32 at middle sizes, microseconds per step for the best one-step
+// shape and the two of these: 100x90x80 23.5, 17.7, 17.6; 200x144x90 75.0,
+// 68.2, 63.7; 256x60x200 79.9, 77.1, 88.8; 256^3 453.5, 454.9, 525.7.  In
+// binary16 the one-step shapes stay ahead.
+constexpr int side_slot(int i)  // place of a sideways direction among those of its ez
+{
+    int n = 0;
+    for (int k = 1; k < i; ++k) n += ez3(k) == ez3(i) && (ex3(k) != 0 || ey3(k) != 0);
+    return n;
+}
+
+template <typename T, bool FORCE, int BS, int RW, int FLAGS>
+__global__ __launch_bounds__(BS, 4) void k3_step2(Args3 a, const T* __restrict__ src, T* __restrict__ dst,
+                                                  const uint32_t* __restrict__ bits, uint32_t words, uint32_t tiles_x,
+                                                  uint32_t tiles_y, int depth)
+{
+    constexpr int RH = BS / RW;
+    __shared__ T lds[36][BS];  // up: slabs x 4 from 0, level: x 8 from 12, down: x 4 from 28
+    const uint32_t t = (FLAGS & kXcdRemap) ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t tx = t % tiles_x, tyz = t / tiles_x;
+    const int q = (int)threadIdx.x % RW, r = (int)threadIdx.x / RW;
+    const int xr = (int)tx * (RW - 2) - 1 + q, yr = (int)(tyz % tiles_y) * (RH - 2) - 1 + r;
+    const int z0 = (int)(tyz / tiles_y) * depth, z1 = min(z0 + depth, a.nz);
+    // columns beyond the ring of a cut tile do a wrapped column's work; no one reads it
+    const int x = xr > a.nx ? 0 : wrap(xr, a.nx), y = yr > a.ny ? 0 : wrap(yr, a.ny);
+    const bool tile = q > 0 && q < RW - 1 && r > 0 && r < RH - 1 && xr < a.nx && yr < a.ny;
+    const uint32_t xm = x == 0 ? (uint32_t)a.nx - 1u : (uint32_t)x - 1u;
+    const uint32_t xp = x == a.nx - 1 ? 0u : (uint32_t)x + 1u;
+    const uint32_t yrow[3] = {(uint32_t)wrap(y - 1, a.ny), (uint32_t)y, (uint32_t)wrap(y + 1, a.ny)};
+    // Byte offsets in a slab; slab and direction go into a uniform base.
+    auto in_slab = [&](int dx, int dy) {
+        return (yrow[1 + dy] * a.rs + (dx == 0 ? (uint32_t)x : (dx < 0 ? xm : xp))) * (uint32_t)sizeof(T);
+    };
+    auto slab = [&](auto* base, int z, int i) {
+        return base + ((size_t)((uint32_t)z * (uint32_t)a.ny) * a.rs + (size_t)((uint32_t)i * a.pitch));
+    };
+
+    // Solid flags of slab z around the column: bits 3 (dy + 1) + dx + 1.
+    auto near_of = [&](int z) {
+        const char* const base = reinterpret_cast<const char*>(bits + (size_t)((uint32_t)z * (uint32_t)a.ny) * words);
+        uint32_t m = 0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint32_t* const p =
+                reinterpret_cast<const uint32_t*>(base + (yrow[d] * words + ((uint32_t)x >> 5)) * 4u);
+            m |= (__builtin_amdgcn_alignbit(p[1], p[0], (uint32_t)x & 31u) & 7u) << (3 * d);
+        }
+        return m;
+    };
+    // Step 1 of the column's cell of slab z: its loads, and the collision,
+    // rounded to storage.
+    auto load1 = [&](int z, T h[19]) {
+        const int zs[3] = {wrap(z - 1, a.nz), z, wrap(z + 1, a.nz)};
+#pragma unroll
+        for (int i = 0; i < 19; ++i) {
+            const char* const base = reinterpret_cast<const char*>(slab(src, zs[1 - ez3(i)], i));
+            h[i] = *reinterpret_cast<const T*>(base + in_slab(-ex3(i), -ey3(i)));
+        }
+    };
+    auto collide1 = [&](const T h[19], float g[19]) {
+#pragma unroll
+        for (int i = 0; i < 19; ++i) g[i] = Store<T>::from_storage(h[i], a.inv_scale);
+        float rho, ux, uy, uz;
+        moments3<FORCE>(a, g, rho, ux, uy, uz);
+        collide3<FORCE>(a, g, rho, ux, uy, uz);
+#pragma unroll
+        for (int i = 0; i < 19; ++i) g[i] = Store<T>::from_storage(Store<T>::to_storage(g[i], a.scale), a.inv_scale);
+    };
+
+    // First slot of direction i of the slab k turns after z0 - 1.
+    auto slot = [&](int i, int k3, int k2) {
+        return ez3(i) == 1 ? k3 * 4 + side_slot(i) : (ez3(i) == 0 ? 12 + k2 * 8 : 28 + k2 * 4) + side_slot(i);
+    };
+    auto put = [&](const float g[19], int k3, int k2) {
+#pragma unroll
+        for (int i = 1; i < 19; ++i)
+            if (ex3(i) != 0 || ey3(i) != 0) lds[slot(i, k3, k2)][threadIdx.x] = Store<T>::to_storage(g[i], a.scale);
+    };
+
+    T h[19];
+    float g[19];
+    load1(wrap(z0 - 1, a.nz), h);
+    collide1(h, g);
+    put(g, 0, 0);
+    float below5 = g[5];  // straight up, of slab z - 1
+    uint32_t near0 = near_of(wrap(z0 - 1, a.nz));
+    load1(z0, h);
+    collide1(h, g);
+    put(g, 1, 1);
+    float mid0 = g[0], mid5 = g[5], mid6 = g[6];
+    uint32_t near1 = near_of(z0);
+    int k3 = 1, k2 = 1;  // LDS places of slab z
+    load1(wrap(z0 + 1, a.nz), h);
+#pragma unroll 1
+    for (int z = z0; z < z1; ++z) {
+        const int zp = wrap(z + 1, a.nz);
+        const int p3 = k3 == 0 ? 2 : k3 - 1, n3 = k3 == 2 ? 0 : k3 + 1;
+        collide1(h, g);
+        const uint32_t near2 = near_of(zp);
+        __syncthreads();  // the last turn's pulls are done
+        put(g, n3, k2 ^ 1);
+        const float top0 = g[0], top5 = g[5], top6 = g[6];
+        __syncthreads();
+        if (z + 1 < z1) load1(wrap(z + 2, a.nz), h);  // under way during step 2
+        if (tile && !(near1 & 16u)) {
+            float f[19];
+            f[0] = mid0;
+            f[5] = below5;
+            f[6] = top6;
+#pragma unroll
+            for (int i = 1; i < 19; ++i)
+                if (ex3(i) != 0 || ey3(i) != 0)
+                    f[i] = Store<T>::from_storage(
+                        lds[slot(i, p3, ez3(i) == 0 ? k2 : k2 ^ 1)][(int)threadIdx.x - ey3(i) * RW - ex3(i)],
+                        a.inv_scale);
+            const uint32_t near[3] = {near0, near1, near2};
+            const uint32_t any = near0 | near1 | near2;
+            if (any) {
+#pragma unroll
+                for (int i = 1; i < 19; ++i) {  // source x - e_i solid: the own opposite one
+                    if (!((near[1 - ez3(i)] >> (3 * (1 - ey3(i)) + 1 - ex3(i))) & 1u)) continue;
+                    if (i == 5) f[i] = mid6;
+                    else if (i == 6) f[i] = mid5;
+                    else f[i] = Store<T>::from_storage(lds[slot(inv3(i), k3, k2)][threadIdx.x], a.inv_scale);
+                }
+            }
+            float rho, ux, uy, uz;
+            moments3<FORCE>(a, f, rho, ux, uy, uz);
+            collide3<FORCE>(a, f, rho, ux, uy, uz);
+#pragma unroll
+            for (int i = 0; i < 19; ++i)
+                st<(FLAGS & kNtStore) != 0>(reinterpret_cast<T*>(reinterpret_cast<char*>(slab(dst, z, i)) + in_slab(0, 0)),
+                                            Store<T>::to_storage(f[i], a.scale));
+            if (any) {
+                const int zs[3] = {wrap(z - 1, a.nz), z, zp};
+#pragma unroll
+                for (int i = 1; i < 19; ++i) {
+                    const int ex = ex3(i), ey = ey3(i), ez = ez3(i);
+                    if (!((near[1 + ez] >> (3 * (1 + ey) + 1 + ex)) & 1u)) continue;
+                    T* const p = reinterpret_cast<T*>(reinterpret_cast<char*>(slab(dst, zs[1 + ez], inv3(i))) +
+                                                      in_slab(ex, ey));
+                    *p = Store<T>::to_storage(f[i], a.scale);
+                }
+            }
+        }
+        below5 = mid5;
+        mid0 = top0;
+        mid5 = top5;
+        mid6 = top6;
+        near0 = near1;
+        near1 = near2;
+        k3 = n3;
+        k2 ^= 1;
     }
 }
 
@@ -394,7 +570,11 @@ const Variant3 kVariants3[] = {
     {256, 1, kNtStore}, {256, 1, 0}, {128, 1, kNtStore}, {512, 1, kNtStore},
     {1024, 1, kNtStore}, {256, 2, kNtStore}, {64, 4, kNtStore},
     {256, 1, kNtStore | kXcdRemap}, {512, 1, kNtStore | kXcdRemap}, {128, 1, kNtStore | kXcdRemap},
+    // two steps per launch (block, region width, flags)
+    {512, 64, kTwoStep | kXcdRemap}, {1024, 32, kTwoStep | kXcdRemap},
 };
+// the one-step shapes of the steps a two-step shape leaves over
+constexpr int kSingle32 = 3, kSingle16 = 2;
 constexpr int kNumVariants3 = (int)(sizeof(kVariants3) / sizeof(kVariants3[0]));
 
 template <typename T, bool FORCE, int BS, int CPT, int FLAGS>
@@ -404,6 +584,28 @@ hipError_t launch3(const Args3& a, const void* src, void* dst, const uint32_t* b
     const uint32_t rows = (uint32_t)a.ny * (uint32_t)a.nz;
     hipLaunchKernelGGL((k3_step<T, FORCE, BS, CPT, FLAGS>), dim3(nseg * rows), dim3(BS), 0, s, a, (const T*)src,
                        (T*)dst, bits, words, nseg);
+    return hipGetLastError();
+}
+
+template <typename T, bool FORCE, int BS, int RW, int FLAGS>
+hipError_t launch3_two(const Args3& a, const void* src, void* dst, const uint32_t* bits, uint32_t words, hipStream_t s)
+{
+    constexpr int RH = BS / RW;
+    const uint32_t tx = (uint32_t)((a.nx + RW - 3) / (RW - 2)), ty = (uint32_t)((a.ny + RH - 3) / (RH - 2));
+    // Chunks of slabs: the number that gives the fewest turns, two more than
+    // its slabs to a chunk, over the rounds its blocks take on the chip.
+    const uint32_t resident = 256u * (1024u / BS);
+    uint32_t tz = 1;
+    uint64_t best = ~0ull;
+    for (uint32_t n = 1; n <= (uint32_t)a.nz && n <= 64; ++n) {
+        const uint32_t d = ((uint32_t)a.nz + n - 1) / n;
+        const uint64_t cost = (uint64_t)((tx * ty * n + resident - 1) / resident) * (d + 2);
+        if (cost < best) best = cost, tz = n;
+    }
+    const int depth = (int)(((uint32_t)a.nz + tz - 1) / tz);
+    tz = (uint32_t)((a.nz + depth - 1) / depth);
+    hipLaunchKernelGGL((k3_step2<T, FORCE, BS, RW, FLAGS>), dim3(tx * ty * tz), dim3(BS), 0, s, a, (const T*)src,
+                       (T*)dst, bits, words, tx, ty, depth);
     return hipGetLastError();
 }
 
@@ -423,6 +625,8 @@ hipError_t dispatch3(int v, const Args3& a, const void* src, void* dst, const ui
     case 7: return launch3<T, FORCE, 256, 1, S | kXcdRemap>(a, src, dst, bits, words, s);
     case 8: return launch3<T, FORCE, 512, 1, S | kXcdRemap>(a, src, dst, bits, words, s);
     case 9: return launch3<T, FORCE, 128, 1, S | kXcdRemap>(a, src, dst, bits, words, s);
+    case 10: return launch3_two<T, FORCE, 512, 64, kXcdRemap>(a, src, dst, bits, words, s);
+    case 11: return launch3_two<T, FORCE, 1024, 32, kXcdRemap>(a, src, dst, bits, words, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -467,6 +671,7 @@ struct lbm3d_handle {
     double* red = nullptr;
     int cur = 0;
     int variant = 0;
+    bool auto_shape = true;  // no shape chosen by the caller: run_variant3's
     int graph_chunk = 100;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -515,10 +720,51 @@ hipError_t prime3(lbm3d_handle* h, int b)
     return hipGetLastError();
 }
 
-hipError_t enqueue_step3(lbm3d_handle* h, int swap)
+// Steps one launch of a shape advances.
+int steps3(int variant) { return (kVariants3[variant].flags & kTwoStep) ? 2 : 1; }
+
+// Whether a shape can step the lattice: the two-step kernel addresses a slab
+// with 32-bit byte offsets.
+bool variant3_ok(const lbm3d_handle* h, int variant)
 {
-    return launch_step3(h->variant, h->f16, h->force, h->a, h->buf[swap], h->buf[swap ^ 1], h->bits, h->words,
-                        h->stream);
+    return steps3(variant) == 1 || (uint64_t)h->a.rs * (uint64_t)h->a.ny * h->elem < (1ull << 32);
+}
+
+// The shape a run takes: the caller's, else 256 threads with plain stores (1)
+// where both buffers fit the 256 MB Infinity Cache, so that the next step
+// finds them there, and non-temporal ones (0) beyond.  Microseconds per step
+// with 0 and 1: binary32 64^3 (40 MB) 11.1 and 9.1, 100x90x80 (115 MB) 26.5
+// and 23.5, 200x144x90 (410 MB) 75 and 93; binary16 200x144x90 (205 MB) 55.1
+// and 42.3, 256x60x200 (233 MB) 49.7 and 40.7, 256^3 (1.3 GB) 268 and 275.
+int run_variant3(const lbm3d_handle* h)
+{
+    if (!h->auto_shape) return h->variant;
+    return 2 * h->elems * h->elem <= (256ull << 20) ? 1 : 0;
+}
+
+// One launch of a shape from buffer `swap` into the other.
+hipError_t enqueue_launch3(lbm3d_handle* h, int variant, int swap)
+{
+    return launch_step3(variant, h->f16, h->force, h->a, h->buf[swap], h->buf[swap ^ 1], h->bits, h->words, h->stream);
+}
+
+// n steps from the current buffer.  Two-step launches go in pairs and the
+// steps left over one by one, so the populations end in the buffer that one
+// launch per step ends in.
+hipError_t enqueue_steps3(lbm3d_handle* h, int n)
+{
+    hipError_t e = hipSuccess;
+    const int v = run_variant3(h);
+    int left = n;
+    if (steps3(v) == 2) {
+        for (; left >= 4 && e == hipSuccess; left -= 4) {
+            e = enqueue_launch3(h, v, h->cur);
+            if (e == hipSuccess) e = enqueue_launch3(h, v, h->cur ^ 1);
+        }
+    }
+    for (; left > 0 && e == hipSuccess; --left, h->cur ^= 1)
+        e = enqueue_launch3(h, steps3(v) == 1 ? v : (h->f16 ? kSingle16 : kSingle32), h->cur);
+    return e;
 }
 
 int ensure_graph3(lbm3d_handle* h, int b)
@@ -526,7 +772,9 @@ int ensure_graph3(lbm3d_handle* h, int b)
     if (h->graph[b]) return LBM_OK;
     TRY3(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     hipError_t le = hipSuccess;
-    for (int s = 0; s < h->graph_chunk && le == hipSuccess; ++s) le = enqueue_step3(h, (b + s) & 1);
+    h->cur = b;
+    le = enqueue_steps3(h, h->graph_chunk);
+    h->cur = b;  // an even number of launches
     hipGraph_t g = nullptr;
     hipError_t ee = hipStreamEndCapture(h->stream, &g);
     if (le != hipSuccess || ee != hipSuccess) {
@@ -553,10 +801,7 @@ int enqueue_run3(lbm3d_handle* h, int nsteps)
             left -= h->graph_chunk;  // an even chunk ends in the buffer it started from
         }
     }
-    for (int s = 0; s < left; ++s) {
-        TRY3(enqueue_step3(h, h->cur));
-        h->cur ^= 1;
-    }
+    TRY3(enqueue_steps3(h, left));
     return LBM_OK;
 }
 
@@ -815,8 +1060,10 @@ int lbm3d_set_variant(lbm3d_handle* h, int variant)
     if (rc) return rc;
     if (variant < 0 || variant >= kNumVariants3) return lbm_fail(LBM_ERR_INVALID, "no 3-D variant %d", variant);
     TRY3(hipStreamSynchronize(h->stream));
-    if (variant != h->variant) drop_graphs3(h);
+    if (!variant3_ok(h, variant)) return lbm_fail(LBM_ERR_INVALID, "3-D variant %d does not fit the lattice", variant);
+    if (variant != h->variant || h->auto_shape) drop_graphs3(h);
     h->variant = variant;
+    h->auto_shape = false;
     return LBM_OK;
 }
 
@@ -852,16 +1099,17 @@ int lbm3d_autotune(lbm3d_handle* h, int steps, int* best_variant, double* ms_per
     int best = v0;
     double best_ms = 1e300;
     for (int v = 0; v < kNumVariants3 && e == hipSuccess; ++v) {
-        h->variant = v;
-        for (int s = 0; s < 2 && e == hipSuccess; ++s, h->cur ^= 1) e = enqueue_step3(h, h->cur);
+        if (!variant3_ok(h, v)) continue;
+        const int per = steps3(v), launches = (steps + per - 1) / per;
+        for (int s = 0; s < 2 && e == hipSuccess; ++s, h->cur ^= 1) e = enqueue_launch3(h, v, h->cur);
         if (e == hipSuccess) e = hipEventRecord(h->ev0, h->stream);
-        for (int s = 0; s < steps && e == hipSuccess; ++s, h->cur ^= 1) e = enqueue_step3(h, h->cur);
+        for (int s = 0; s < launches && e == hipSuccess; ++s, h->cur ^= 1) e = enqueue_launch3(h, v, h->cur);
         if (e == hipSuccess) e = hipEventRecord(h->ev1, h->stream);
         if (e == hipSuccess) e = hipEventSynchronize(h->ev1);
         float t = 0.0f;
         if (e == hipSuccess) e = hipEventElapsedTime(&t, h->ev0, h->ev1);
-        if (e == hipSuccess && t / steps < best_ms * kTuneMargin) {
-            best_ms = t / steps;
+        if (e == hipSuccess && t / (launches * per) < best_ms * kTuneMargin) {
+            best_ms = t / (launches * per);
             best = v;
         }
     }
@@ -869,8 +1117,9 @@ int lbm3d_autotune(lbm3d_handle* h, int steps, int* best_variant, double* ms_per
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     (void)hipFree(saved);
     h->cur = cur0;
-    if (best != v0) drop_graphs3(h);
+    if (best != v0 || h->auto_shape) drop_graphs3(h);
     h->variant = best;
+    h->auto_shape = false;
     if (e != hipSuccess) return lbm_fail(LBM_ERR_HIP, "3-D autotune: %s", hipGetErrorString(e));
     if (best_variant) *best_variant = best;
     if (ms_per_step) *ms_per_step = best_ms;

@@ -752,8 +752,9 @@ class Lattice3D:
 
 
 def variant3_shapes() -> list[tuple[int, int, int]]:
-    """(threads per block, cells per thread, flags: 1 non-temporal stores)
-    of the D3Q19 step kernel's shapes."""
+    """(threads per block, cells per thread, flags: 1 non-temporal stores, 4
+    rows per XCD, 16 two steps per launch, with the region's width in place of
+    the cells per thread) of the D3Q19 step kernels' shapes."""
     lib = load_library()
     out = []
     for v in range(lib.lbm3d_variant_count()):
