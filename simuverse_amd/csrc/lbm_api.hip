@@ -499,8 +499,7 @@ int lbm_create(const lbm_desc* desc, lbm_handle** out)
         free_handle(h);
         return fail(LBM_ERR_HIP, "stream/event setup: %s", hipGetErrorString(e));
     }
-    // a frame's readback finds its slots ready; larger ones add theirs when they come
-    (void)h->staging.reserve(std::min<size_t>(12 * n, 2u << 20));
+    (void)h->staging.reserve(12 * n);  // of the macro fields
     rc = do_reset(h);
     if (rc != LBM_OK) {
         std::string msg = g_last_error;

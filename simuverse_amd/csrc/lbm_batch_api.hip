@@ -348,6 +348,7 @@ int lbm_batch_create(const lbm_domain_desc* domains, int count, int storage, lbm
         batch_free(b);
         return rc;
     }
+    (void)b->staging.reserve((size_t)12 * b->max_cells);  // of the largest domain's macro fields
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
@@ -499,8 +500,6 @@ int lbm_batch_macro(lbm_batch* b, int d, float* rho, float* ux, float* uy)
     float* v = u + n;
     BATCH_TRY(launch_phys_macro(b->f16, b->dom[d].x_edge, b->dom[d].force != 0, b->args(d), b->view(b->cur, d),
                                 b->mat + b->cell_off[d], r, u, v, b->stream));
-    // room for the largest domain at once: a program reads them one after the other
-    (void)b->staging.reserve((size_t)3 * b->max_cells * sizeof(float));
     const size_t nb = n * sizeof(float);
     const HostPiece p[3] = {{rho, r, nb}, {ux, u, nb}, {uy, v, nb}};
     BATCH_TRY(b->staging.to_host(p, 3, b->stream, b->dev));

@@ -41,11 +41,12 @@ public:
         if (host_) (void)hipHostFree(host_);
     }
 
-    // Pinned memory for readbacks of up to `total` bytes at a time (at most
-    // kSlots * kSlot of it); kept until the object ends.
+    // Pinned memory for readbacks of `total` bytes at a time, kept until the
+    // object ends; called where the object is made, so that the first readback
+    // finds it (12 MiB take about 2 ms to pin).
     hipError_t reserve(size_t total)
     {
-        const size_t want = std::min(kSlots, (total + kSlot - 1) / kSlot);
+        const size_t want = std::min(slots_for(total), (total + kSlot - 1) / kSlot);
         for (size_t k = 0; k < want; ++k)
             if (!events_[k])
                 if (hipError_t r = hipEventCreateWithFlags(&events_[k], hipEventDisableTiming)) return r;
@@ -53,7 +54,11 @@ public:
         if (host_) (void)hipHostFree(host_);
         host_ = nullptr;
         slots_ = 0;
-        if (hipError_t r = hipHostMalloc((void**)&host_, want * kSlot, hipHostMallocDefault)) return r;
+        if (hipError_t r = hipHostMalloc((void**)&host_, want * kSlot, hipHostMallocDefault)) {
+            host_ = nullptr;
+            (void)hipGetLastError();  // readbacks go the runtime's way
+            return r;
+        }
         slots_ = want;
         return hipSuccess;
     }
@@ -100,9 +105,14 @@ private:
         size_t at, bytes;        // in the run
     };
     static constexpr size_t kSlots = 12, kSlot = 1u << 20;
-    // From here threads are faster also into warm pages: 10.8 MB 0.45 ms on
-    // one thread and 1.05 on twelve, 19 MB 1.4 and 1.1.
+    // Below 16 MiB one thread and two slots that take turns (the link fills one
+    // faster than the thread empties the other; 10.8 MB into warm pages 0.45 ms,
+    // and 1.05 ms with twelve threads), four threads up to 32 MiB, twelve beyond.
     static constexpr size_t kThreaded = 16u << 20;
+    static constexpr size_t slots_for(size_t total)
+    {
+        return total < kThreaded ? 2 : (total < 2 * kThreaded ? 4 : kSlots);
+    }
 
     // Memory the runtime has pinned or owns is written directly.
     static bool known_to_runtime(const void* p)
