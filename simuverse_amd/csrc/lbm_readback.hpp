@@ -105,13 +105,15 @@ private:
         size_t at, bytes;        // in the run
     };
     static constexpr size_t kSlots = 12, kSlot = 1u << 20;
-    // Below 16 MiB one thread and two slots that take turns (the link fills one
-    // faster than the thread empties the other; 10.8 MB into warm pages 0.45 ms,
-    // and 1.05 ms with twelve threads), four threads up to 32 MiB, twelve beyond.
-    static constexpr size_t kThreaded = 16u << 20;
+    // Below 6 MiB one thread and two slots that take turns (the link fills one
+    // faster than the thread empties the other), four threads up to 32 MiB,
+    // twelve beyond.  One thread and four, microseconds, a program's arrays
+    // reused and kept: 5.0 MB 250 to 1180 and 600 to 750; 6.7 MB 1040 to 1400
+    // and 720 to 800; 12.6 MB 1490 to 1880 and 900.
+    static constexpr size_t kThreaded = 6u << 20, kMore = 32u << 20;
     static constexpr size_t slots_for(size_t total)
     {
-        return total < kThreaded ? 2 : (total < 2 * kThreaded ? 4 : kSlots);
+        return total < kThreaded ? 2 : (total < kMore ? 4 : kSlots);
     }
 
     // Memory the runtime has pinned or owns is written directly.

@@ -10,9 +10,9 @@ from simuverse_amd import workloads as W
 pytestmark = pytest.mark.gpu
 
 # 12 n bytes of macro fields: under one slot of 1 MiB; pieces that straddle
-# slots; more chunks than slots; just under and from the 16 MiB on where four
-# threads start, and over the 32 MiB where twelve do
-SIZES = [(3, 3), (300, 291), (600, 375), (1195, 1170), (1024, 1365), (1024, 1366), (1531, 1037), (1700, 1650)]
+# slots; two slots in turn; just under and from the 6 MiB on where four threads
+# start; more chunks than slots; just under and over the 32 MiB where twelve do
+SIZES = [(3, 3), (300, 291), (600, 375), (1024, 511), (1024, 512), (1531, 1037), (1700, 1644), (1700, 1650)]
 
 
 @pytest.mark.parametrize("nx, ny", SIZES)
