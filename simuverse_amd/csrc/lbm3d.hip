@@ -107,8 +107,13 @@ __device__ inline void moments3(const Args3& a, const float g[19], float& rho, f
     }
 }
 
-// BGK + Guo in deviation form, as the 2-D phys_collide.
-template <bool FORCE>
+// BGK + Guo in deviation form, as the 2-D phys_collide.  fa and fb flip sign
+// with the direction; with PAIRED the odd ones of each pair serve both, which
+// leaves the two-step kernel 18 scalar registers.  The one-step kernel reads
+// each direction's own: its 38 constants lie side by side and come in ten
+// scalar loads, where every other one takes 24 and waits for them (float,
+// 24x200x100 with force: 29.9 and 32.1 us per step; 160^3: 103.8 and 107.1).
+template <bool FORCE, bool PAIRED>
 __device__ inline void collide3(const Args3& a, float g[19], float rho, float ux, float uy, float uz)
 {
     const float dr = rho - 1.0f;
@@ -126,8 +131,7 @@ __device__ inline void collide3(const Args3& a, float g[19], float rho, float ux
         const float q = fmaf(eu, fmaf(4.5f, eu, 3.0f), -usq);
         const float geq = fmaf(wr[k], q, wd[k]);
         float out = fmaf(-a.omega, g[i] - geq, g[i]);
-        // fa and fb flip sign with the direction: the odd ones of each pair serve both
-        if (FORCE && (i == 0 || (i & 1))) out += fmaf(a.fb[i], eu, fmaf(-a.fc[k], ug, a.fa[i]));
+        if (FORCE && (!PAIRED || i == 0 || (i & 1))) out += fmaf(a.fb[i], eu, fmaf(-a.fc[k], ug, a.fa[i]));
         else if (FORCE) out += fmaf(-a.fb[i - 1], eu, fmaf(-a.fc[k], ug, -a.fa[i - 1]));
         g[i] = out;
     }
@@ -188,7 +192,7 @@ __device__ inline void cell3(const Args3& a, const T* __restrict__ src, T* __res
     }
     float rho, ux, uy, uz;
     moments3<FORCE>(a, g, rho, ux, uy, uz);
-    collide3<FORCE>(a, g, rho, ux, uy, uz);
+    collide3<FORCE, false>(a, g, rho, ux, uy, uz);
 #pragma unroll
     for (int i = 0; i < 19; ++i)
         st<(FLAGS & kNtStore) != 0>(elem3(dst, a, nb.row[1][1], i, (uint32_t)x), Store<T>::to_storage(g[i], a.scale));
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(BS, 4) void k3_step2(Args3 a, const T* __restrict__
         for (int i = 0; i < 19; ++i) g[i] = Store<T>::from_storage(h[i], a.inv_scale);
         float rho, ux, uy, uz;
         moments3<FORCE>(a, g, rho, ux, uy, uz);
-        collide3<FORCE>(a, g, rho, ux, uy, uz);
+        collide3<FORCE, true>(a, g, rho, ux, uy, uz);
 #pragma unroll
         for (int i = 0; i < 19; ++i) g[i] = Store<T>::from_storage(Store<T>::to_storage(g[i], a.scale), a.inv_scale);
     };
@@ -373,7 +377,7 @@ __global__ __launch_bounds__(BS, 4) void k3_step2(Args3 a, const T* __restrict__
             }
             float rho, ux, uy, uz;
             moments3<FORCE>(a, f, rho, ux, uy, uz);
-            collide3<FORCE>(a, f, rho, ux, uy, uz);
+            collide3<FORCE, true>(a, f, rho, ux, uy, uz);
 #pragma unroll
             for (int i = 0; i < 19; ++i)
                 st<(FLAGS & kNtStore) != 0>(reinterpret_cast<T*>(reinterpret_cast<char*>(slab(dst, z, i)) + in_slab(0, 0)),
