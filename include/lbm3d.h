@@ -81,8 +81,9 @@ int lbm3d_variant_count(void);
  * two steps per launch, streamed along z, with cells_per_thread the width of
  * a block's region (one slab must lie under 4 GiB; launches go in pairs, the
  * steps left over run one per launch).  Until a shape is chosen, lbm3d_run
- * takes 256 threads with plain stores where both buffers fit the 256 MB
- * cache and with non-temporal ones beyond. */
+ * takes 256 threads with plain stores where the next step finds both buffers
+ * in a cache (under 7 MiB, and from 29 to 256) and with non-temporal ones
+ * elsewhere. */
 int lbm3d_variant_info(int variant, int* block, int* cells_per_thread, int* flags);
 int lbm3d_set_variant(lbm3d_handle* h, int variant);
 int lbm3d_get_variant(lbm3d_handle* h, int* variant);

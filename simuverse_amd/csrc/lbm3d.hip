@@ -734,16 +734,11 @@ bool variant3_ok(const lbm3d_handle* h, int variant)
     return steps3(variant) == 1 || (uint64_t)h->a.rs * (uint64_t)h->a.ny * h->elem < (1ull << 32);
 }
 
-// The shape a run takes: the caller's, else 256 threads with plain stores (1)
-// where both buffers fit the 256 MB Infinity Cache, so that the next step
-// finds them there, and non-temporal ones (0) beyond.  Microseconds per step
-// with 0 and 1: binary32 64^3 (40 MB) 11.1 and 9.1, 100x90x80 (115 MB) 26.5
-// and 23.5, 200x144x90 (410 MB) 75 and 93; binary16 200x144x90 (205 MB) 55.1
-// and 42.3, 256x60x200 (233 MB) 49.7 and 40.7, 256^3 (1.3 GB) 268 and 275.
+// The shape a run takes: the caller's, else default_variant3's.
 int run_variant3(const lbm3d_handle* h)
 {
     if (!h->auto_shape) return h->variant;
-    return 2 * h->elems * h->elem <= (256ull << 20) ? 1 : 0;
+    return default_variant3(2 * h->elems * h->elem);
 }
 
 // One launch of a shape from buffer `swap` into the other.

@@ -52,6 +52,24 @@ inline bool nstep_fits(int bw, int ns, int nx, int ny, int xedge)
 {
     return nx >= ns && ny >= ns && two_step_fits(bw, nx, ny, xedge);
 }
+// The 3-D shape for a lattice whose caller chose none, by the bytes of both
+// population buffers: 256 threads with plain stores (1), whose lines the next
+// step finds in the caches, or with non-temporal ones (0).  Beyond the 256 MB
+// Infinity Cache the lines are gone before they are read, and where the two
+// buffers fill most of the eight 4 MB L2 caches plain stores push out what the
+// step still has to read.  Microseconds per step with 0 and 1 without force
+// (with force they order the same way):
+//   binary32  32^3 4.75 MiB 3.76, 3.55;  128x16x24 7.1 4.12, 3.90;  36^3 9.0 5.35, 5.43;
+//             48^3 16.0 5.88, 6.40;  52^3 25.1 8.16, 8.68;  256x256x3 28.5 7.49, 7.85;
+//             56^3 29.1 8.35, 7.68;  64^3 38 9.41, 8.13;  128x128x100 238 42.1, 31.1;
+//             160^3 594 102, 107
+//   binary16  44^3 6.74 MiB 5.80, 5.65;  16x128x48 7.1 8.96, 9.65;  52^3 12.5 6.59, 6.80;
+//             64^3 19.0 7.23, 7.78;  72^3 30.1 13.1, 11.4;  256x60x200 222 45.9, 32.0;  160^3 297 72.5, 78.0
+constexpr int default_variant3(uint64_t bytes)
+{
+    const uint64_t mib = bytes >> 20;
+    return mib < 7 || (mib >= 29 && bytes <= (256ull << 20)) ? 1 : 0;
+}
 // Blocks of bs threads for n work items.
 inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
