@@ -17,7 +17,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -148,7 +150,12 @@ private:
     hipError_t take(const Chunk& c, size_t k)
     {
         hipError_t e = hipEventSynchronize(events_[k]);
-        if (e != hipSuccess) return e;
+        if (e == hipSuccess) unload(c, k);
+        return e;
+    }
+
+    void unload(const Chunk& c, size_t k)
+    {
         const char* from = host_ + k * kSlot;
         size_t at = c.at, left = c.bytes;
         for (const HostPiece* p = c.first; left; at = at > p->bytes ? at - p->bytes : 0, ++p) {
@@ -158,7 +165,6 @@ private:
             from += n;
             left -= n;
         }
-        return e;
     }
 
     hipError_t pipelined(const std::vector<Chunk>& chunks, hipStream_t s)
@@ -178,28 +184,49 @@ private:
         return e != hipSuccess ? e : w;
     }
 
+    // The other threads sleep until the stream has come to the readback: the
+    // runtime's waits spin, and twelve of them through a run of 2000 steps at
+    // 4096^2 took 1.7 s of processor time in 0.14 s.
     hipError_t threaded(const std::vector<Chunk>& chunks, hipStream_t s, int dev)
     {
         const size_t n = chunks.size();
         const size_t hw = std::max(1u, std::thread::hardware_concurrency());
         const size_t workers = std::min({slots_, n, hw});
         std::atomic<int> error{(int)hipSuccess};
-        std::atomic<size_t> next{0};
-        auto work = [&](size_t w) {
-            hipError_t e = hipSetDevice(dev);
+        std::atomic<size_t> next{1};  // chunk 0 is the calling thread's
+        std::mutex gate;
+        std::condition_variable opened;
+        bool open = false;
+        auto rest = [&](size_t w, hipError_t e) {
             for (size_t k; e == hipSuccess && error.load() == (int)hipSuccess && (k = next.fetch_add(1)) < n;) {
                 e = issue(chunks[k], w, s);
                 if (e == hipSuccess) e = take(chunks[k], w);
             }
             if (e != hipSuccess) error.store((int)e);
         };
+        auto work = [&](size_t w) {
+            {
+                std::unique_lock<std::mutex> lock(gate);
+                opened.wait(lock, [&] { return open; });
+            }
+            rest(w, hipSetDevice(dev));
+        };
         std::vector<std::thread> threads;
+        hipError_t e = issue(chunks[0], 0, s);
         try {
             threads.reserve(workers);
             for (size_t w = 1; w < workers; ++w) threads.emplace_back(work, w);
         } catch (...) {  // no thread to be had: the ones that started, and this one, do the work
         }
-        work(0);
+        if (e == hipSuccess) e = hipEventSynchronize(events_[0]);
+        if (e != hipSuccess) error.store((int)e);
+        {
+            std::lock_guard<std::mutex> lock(gate);
+            open = true;
+        }
+        opened.notify_all();
+        if (e == hipSuccess) unload(chunks[0], 0);
+        rest(0, e);
         for (std::thread& t : threads) t.join();
         const hipError_t w = hipStreamSynchronize(s);
         return error.load() != (int)hipSuccess ? (hipError_t)error.load() : w;
