@@ -19,7 +19,11 @@
  *   - Every function returns an int status: LBM_OK (0) or an LBM_ERR_* code.
  *     Nothing aborts or throws across the ABI; lbm_last_error() returns the
  *     message of the last failure on the calling thread.
- *   - The caller owns host memory, the library owns device memory.
+ *   - The caller owns host memory, the library owns device memory.  Fields and
+ *     populations read back into ordinary memory go through up to 12 MiB of
+ *     pinned memory per device, which the handles of every kind share; the
+ *     first readback takes it and the last of those handles to be destroyed
+ *     gives it back.
  *   - Each handle owns one HIP stream; calls on one handle are stream
  *     ordered.  A handle is not thread-safe; separate handles may be driven
  *     from separate threads.

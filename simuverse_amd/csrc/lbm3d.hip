@@ -889,7 +889,6 @@ int lbm3d_create(const lbm3d_desc* desc, lbm3d_handle** out)
         free3(h);
         return lbm_fail(rc, "%s", msg.c_str());
     }
-    (void)h->staging.reserve(16 * h->cells);  // of the macro fields
     *out = h;
     return LBM_OK;
 }

@@ -499,7 +499,6 @@ int lbm_create(const lbm_desc* desc, lbm_handle** out)
         free_handle(h);
         return fail(LBM_ERR_HIP, "stream/event setup: %s", hipGetErrorString(e));
     }
-    (void)h->staging.reserve(12 * n);  // of the macro fields
     rc = do_reset(h);
     if (rc != LBM_OK) {
         std::string msg = g_last_error;

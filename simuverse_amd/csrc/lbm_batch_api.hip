@@ -348,7 +348,6 @@ int lbm_batch_create(const lbm_domain_desc* domains, int count, int storage, lbm
         batch_free(b);
         return rc;
     }
-    (void)b->staging.reserve((size_t)12 * b->max_cells);  // of the largest domain's macro fields
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);

@@ -6,10 +6,10 @@
 // memory in 27 us (57 GB/s for large copies).  Fresh host pages are the other
 // bound: one thread fills them at 4 GB/s where the kernel has to clear them.
 //
-// Staging keeps a few pinned slots with the handle.  A small readback
-// pipelines its chunks through them on the calling thread; a large one
-// starts threads that take chunks through a slot of their own each and end
-// before the call returns.  4096^2: 7.1 ms, 2048^2: 5.6 to 2.0 ms.
+// Staging copies through pinned slots, which the objects on a device share.  A
+// small readback pipelines its chunks through them on the calling thread; a
+// large one starts threads that take chunks through a slot of their own each
+// and end before the call returns.  4096^2: 6.9 ms, 2048^2: 4.6 to 1.9 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -21,6 +21,7 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 namespace lbm {
@@ -31,6 +32,91 @@ struct HostPiece {
     size_t bytes;
 };
 
+// The pinned slots of one device: at most kSlots of 1 MiB, made when a
+// readback first asks for them, lent for the length of one call, and freed
+// with the last object that read back through them.  Pinning is what costs
+// (0.2 ms a slot, once), so objects do not keep their own: a program with a
+// thousand lattices pins as much as one with a single one.
+class SlotPool {
+public:
+    static constexpr size_t kSlots = 12, kSlot = 1u << 20;
+    struct Slot {
+        char* host = nullptr;
+        hipEvent_t event = nullptr;
+    };
+
+    // nullptr: a device number beyond the table, whose readbacks go the
+    // runtime's way
+    static SlotPool* of(int dev)
+    {
+        static SlotPool pools[64];
+        return dev >= 0 && dev < 64 ? &pools[dev] : nullptr;
+    }
+
+    void attach()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        ++users_;
+    }
+    void detach()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (--users_) return;
+        for (; made_; --made_) (void)hipEventDestroy(slots_[made_ - 1].event);
+        for (; blocks_; --blocks_) (void)hipHostFree(block_[blocks_ - 1]);
+    }
+
+    // Lends up to `want` slots; fewer, or none, where other threads hold them
+    // or memory cannot be pinned.
+    size_t lend(Slot** out, size_t want)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t n = 0, idle = 0;
+        for (size_t k = 0; k < made_; ++k) idle += !lent_[k];
+        if (idle < want) grow(std::min(want - idle, kSlots - made_));
+        for (size_t k = 0; k < made_ && n < want; ++k) {
+            if (lent_[k]) continue;
+            lent_[k] = true;
+            out[n++] = &slots_[k];
+        }
+        return n;
+    }
+    void take_back(Slot* const* in, size_t n)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (size_t k = 0; k < n; ++k) lent_[in[k] - slots_] = false;
+    }
+
+private:
+    // More slots, side by side in one allocation (single ones of 1 MiB take 3 %
+    // longer to fill); none if there is no memory to pin.
+    void grow(size_t count)
+    {
+        char* host = nullptr;
+        if (count == 0) return;
+        if (hipHostMalloc((void**)&host, count * kSlot, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();  // the readback goes the runtime's way
+            return;
+        }
+        const size_t before = made_;
+        for (; count; --count, ++made_, host += kSlot) {
+            Slot& s = slots_[made_];
+            if (hipEventCreateWithFlags(&s.event, hipEventDisableTiming) != hipSuccess) break;
+            s.host = host;
+        }
+        if (count) (void)hipGetLastError();
+        if (made_ > before) block_[blocks_++] = slots_[before].host;
+        else (void)hipHostFree(host);
+    }
+
+    std::mutex mu_;
+    size_t users_ = 0, made_ = 0, blocks_ = 0;
+    Slot slots_[kSlots];
+    bool lent_[kSlots] = {};
+    char* block_[kSlots] = {};
+};
+static_assert(std::is_trivially_destructible_v<SlotPool>, "usable while a process ends");
+
 class Staging {
 public:
     Staging() = default;
@@ -38,31 +124,7 @@ public:
     Staging& operator=(const Staging&) = delete;
     ~Staging()
     {
-        for (hipEvent_t e : events_)
-            if (e) (void)hipEventDestroy(e);
-        if (host_) (void)hipHostFree(host_);
-    }
-
-    // Pinned memory for readbacks of `total` bytes at a time, kept until the
-    // object ends; called where the object is made, so that the first readback
-    // finds it (12 MiB take about 2 ms to pin).
-    hipError_t reserve(size_t total)
-    {
-        const size_t want = std::min(slots_for(total), (total + kSlot - 1) / kSlot);
-        for (size_t k = 0; k < want; ++k)
-            if (!events_[k])
-                if (hipError_t r = hipEventCreateWithFlags(&events_[k], hipEventDisableTiming)) return r;
-        if (want <= slots_) return hipSuccess;
-        if (host_) (void)hipHostFree(host_);
-        host_ = nullptr;
-        slots_ = 0;
-        if (hipError_t r = hipHostMalloc((void**)&host_, want * kSlot, hipHostMallocDefault)) {
-            host_ = nullptr;
-            (void)hipGetLastError();  // readbacks go the runtime's way
-            return r;
-        }
-        slots_ = want;
-        return hipSuccess;
+        if (pool_) pool_->detach();
     }
 
     // Copies the pieces, in stream order after what `s` holds, and waits.
@@ -86,7 +148,8 @@ private:
             direct = direct || known_to_runtime(pieces[k].dst);
         }
         if (total == 0) return hipStreamSynchronize(s);
-        if (direct || reserve(total) != hipSuccess) return plain(pieces, count, s);
+        if (direct) return plain(pieces, count, s);
+        if (!pool_ && (pool_ = SlotPool::of(dev))) pool_->attach();
         std::vector<Chunk> chunks;
         for (int k = 0; k < count;) {
             // a run of pieces that lie one behind the other on the device
@@ -99,14 +162,29 @@ private:
                 chunks.push_back({pieces + k, at, std::min(kSlot, run - at)});
             k = end;
         }
-        return total < kThreaded ? pipelined(chunks, s) : threaded(chunks, s, dev);
+        const Loan slots(pool_, std::min(slots_for(total), chunks.size()));
+        if (slots.count == 0) return plain(pieces, count, s);
+        return total < kThreaded ? pipelined(chunks, slots, s) : threaded(chunks, slots, s, dev);
     }
+
+    struct Loan {  // slots of the pool for one call
+        SlotPool* const pool;
+        SlotPool::Slot* slot[SlotPool::kSlots];
+        const size_t count;
+        Loan(SlotPool* p, size_t want) : pool(p), slot{}, count(p ? p->lend(slot, want) : 0) {}
+        Loan(const Loan&) = delete;
+        Loan& operator=(const Loan&) = delete;
+        ~Loan()
+        {
+            if (count) pool->take_back(slot, count);
+        }
+    };
 
     struct Chunk {
         const HostPiece* first;  // of its run
         size_t at, bytes;        // in the run
     };
-    static constexpr size_t kSlots = 12, kSlot = 1u << 20;
+    static constexpr size_t kSlot = SlotPool::kSlot;
     // Below 6 MiB one thread and two slots that take turns (the link fills one
     // faster than the thread empties the other), four threads up to 32 MiB,
     // twelve beyond.  One thread and four, microseconds, a program's arrays
@@ -115,7 +193,7 @@ private:
     static constexpr size_t kThreaded = 6u << 20, kMore = 32u << 20;
     static constexpr size_t slots_for(size_t total)
     {
-        return total < kThreaded ? 2 : (total < kMore ? 4 : kSlots);
+        return total < kThreaded ? 2 : (total < kMore ? 4 : SlotPool::kSlots);
     }
 
     // Memory the runtime has pinned or owns is written directly.
@@ -140,23 +218,22 @@ private:
         return hipStreamSynchronize(s);
     }
 
-    hipError_t issue(const Chunk& c, size_t k, hipStream_t s)
+    static hipError_t issue(const Chunk& c, const SlotPool::Slot& slot, hipStream_t s)
     {
-        hipError_t e = hipMemcpyAsync(host_ + k * kSlot, (const char*)c.first->src + c.at, c.bytes,
-                                      hipMemcpyDeviceToHost, s);
-        return e == hipSuccess ? hipEventRecord(events_[k], s) : e;
+        hipError_t e = hipMemcpyAsync(slot.host, (const char*)c.first->src + c.at, c.bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipEventRecord(slot.event, s) : e;
     }
 
-    hipError_t take(const Chunk& c, size_t k)
+    static hipError_t take(const Chunk& c, const SlotPool::Slot& slot)
     {
-        hipError_t e = hipEventSynchronize(events_[k]);
-        if (e == hipSuccess) unload(c, k);
+        hipError_t e = hipEventSynchronize(slot.event);
+        if (e == hipSuccess) unload(c, slot);
         return e;
     }
 
-    void unload(const Chunk& c, size_t k)
+    static void unload(const Chunk& c, const SlotPool::Slot& slot)
     {
-        const char* from = host_ + k * kSlot;
+        const char* from = slot.host;
         size_t at = c.at, left = c.bytes;
         for (const HostPiece* p = c.first; left; at = at > p->bytes ? at - p->bytes : 0, ++p) {
             if (at >= p->bytes) continue;
@@ -167,17 +244,17 @@ private:
         }
     }
 
-    hipError_t pipelined(const std::vector<Chunk>& chunks, hipStream_t s)
+    static hipError_t pipelined(const std::vector<Chunk>& chunks, const Loan& slots, hipStream_t s)
     {
         const size_t n = chunks.size();
         hipError_t e = hipSuccess;
         size_t issued = 0, taken = 0;
         while (taken < n && e == hipSuccess) {
-            while (e == hipSuccess && issued < n && issued < taken + slots_) {
-                e = issue(chunks[issued], issued % slots_, s);
+            while (e == hipSuccess && issued < n && issued < taken + slots.count) {
+                e = issue(chunks[issued], *slots.slot[issued % slots.count], s);
                 if (e == hipSuccess) ++issued;
             }
-            if (e == hipSuccess) e = take(chunks[taken], taken % slots_);
+            if (e == hipSuccess) e = take(chunks[taken], *slots.slot[taken % slots.count]);
             ++taken;
         }
         const hipError_t w = hipStreamSynchronize(s);  // no copy into a slot outlives the call
@@ -187,11 +264,11 @@ private:
     // The other threads sleep until the stream has come to the readback: the
     // runtime's waits spin, and twelve of them through a run of 2000 steps at
     // 4096^2 took 1.7 s of processor time in 0.14 s.
-    hipError_t threaded(const std::vector<Chunk>& chunks, hipStream_t s, int dev)
+    static hipError_t threaded(const std::vector<Chunk>& chunks, const Loan& slots, hipStream_t s, int dev)
     {
         const size_t n = chunks.size();
         const size_t hw = std::max(1u, std::thread::hardware_concurrency());
-        const size_t workers = std::min({slots_, n, hw});
+        const size_t workers = std::min({slots.count, n, hw});
         std::atomic<int> error{(int)hipSuccess};
         std::atomic<size_t> next{1};  // chunk 0 is the calling thread's
         std::mutex gate;
@@ -199,8 +276,8 @@ private:
         bool open = false;
         auto rest = [&](size_t w, hipError_t e) {
             for (size_t k; e == hipSuccess && error.load() == (int)hipSuccess && (k = next.fetch_add(1)) < n;) {
-                e = issue(chunks[k], w, s);
-                if (e == hipSuccess) e = take(chunks[k], w);
+                e = issue(chunks[k], *slots.slot[w], s);
+                if (e == hipSuccess) e = take(chunks[k], *slots.slot[w]);
             }
             if (e != hipSuccess) error.store((int)e);
         };
@@ -212,29 +289,27 @@ private:
             rest(w, hipSetDevice(dev));
         };
         std::vector<std::thread> threads;
-        hipError_t e = issue(chunks[0], 0, s);
+        hipError_t e = issue(chunks[0], *slots.slot[0], s);
         try {
             threads.reserve(workers);
             for (size_t w = 1; w < workers; ++w) threads.emplace_back(work, w);
         } catch (...) {  // no thread to be had: the ones that started, and this one, do the work
         }
-        if (e == hipSuccess) e = hipEventSynchronize(events_[0]);
+        if (e == hipSuccess) e = hipEventSynchronize(slots.slot[0]->event);
         if (e != hipSuccess) error.store((int)e);
         {
             std::lock_guard<std::mutex> lock(gate);
             open = true;
         }
         opened.notify_all();
-        if (e == hipSuccess) unload(chunks[0], 0);
+        if (e == hipSuccess) unload(chunks[0], *slots.slot[0]);
         rest(0, e);
         for (std::thread& t : threads) t.join();
         const hipError_t w = hipStreamSynchronize(s);
         return error.load() != (int)hipSuccess ? (hipError_t)error.load() : w;
     }
 
-    char* host_ = nullptr;
-    size_t slots_ = 0;
-    hipEvent_t events_[kSlots] = {};
+    SlotPool* pool_ = nullptr;  // from the first readback on
 };
 
 }  // namespace lbm

@@ -97,12 +97,84 @@ static void copy_fails()
         }
 }
 
+// Pinned memory does not grow with the objects, is given back with the last of
+// them, and is not taken before a readback asks for it.
+static void pinned()
+{
+    fake::Stream s;
+    CHECK(fake::pinned == 0);
+    for (int round = 0; round < 2; ++round) {
+        std::vector<std::unique_ptr<Staging>> many;
+        for (int k = 0; k < 200; ++k) many.push_back(std::make_unique<Staging>());
+        CHECK(fake::pinned == 0 && fake::events == 0);
+        reads(*many[0], &s, 1000, false);
+        CHECK(fake::pinned <= MiB);
+        for (auto& st : many) reads(*st, &s, 100000, false);
+        CHECK(fake::pinned <= 2 * MiB);
+        reads(*many[3], &s, 14 * MiB, false);
+        reads(*many[4], &s, 14 * MiB, false);
+        CHECK(fake::pinned <= 12 * MiB);
+        while (many.size() > 1) many.pop_back();
+        reads(*many[0], &s, 3 * MiB, true);
+        many.clear();
+        CHECK(fake::pinned == 0 && fake::events == 0);
+    }
+    CHECK(fake::pinned_most <= 12 * MiB);
+}
+
+// Objects of their own on streams of their own, each driven by one thread, at
+// the same time; one is made and ended again and again.
+static void together()
+{
+    std::vector<std::thread> threads;
+    for (int t = 0; t < 5; ++t)
+        threads.emplace_back([t] {
+            fake::Stream s;
+            std::unique_ptr<Staging> st = std::make_unique<Staging>();
+            for (int k = 0; k < 12; ++k) {
+                const size_t n = (size_t)(1 + (t * 7 + k * 5) % 13) * MiB + 4 * t;
+                std::vector<unsigned> src = device(n, (unsigned)(t + k));
+                std::vector<char> out(n + 1, 77);
+                const HostPiece p{out.data(), src.data(), n};
+                CHECK(st->to_host(&p, 1, &s, t == 4 ? 64 : 0) == hipSuccess);
+                CHECK(std::memcmp(out.data(), src.data(), n) == 0 && out[n] == 77);
+                if (t == 0) st = std::make_unique<Staging>();
+            }
+        });
+    for (std::thread& t : threads) t.join();
+    CHECK(fake::pinned_most <= 12 * MiB);
+    CHECK(fake::pinned == 0 && fake::events == 0);
+}
+
+// Without pinned memory or events the readback goes the runtime's way; with
+// some of them it takes what there is.
+static void short_of_memory()
+{
+    fake::Stream s;
+    for (size_t n : {1000ul, MiB, 3 * MiB, 14 * MiB})
+        for (int good : {0, 1, 5}) {
+            Staging st;
+            if (good) reads(st, &s, (good == 1 ? 1 : 4) * MiB / 4, false);
+            fake::fail_pin = 1000;
+            reads(st, &s, n, false);
+            fake::fail_pin = 0;
+            fake::fail_event = 1;
+            reads(st, &s, n, true);
+            fake::fail_event = 0;
+            reads(st, &s, n, false);
+        }
+    CHECK(fake::pinned == 0 && fake::events == 0);
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") bytes();
     else if (what == "busy") busy();
     else if (what == "copy_fails") copy_fails();
+    else if (what == "pinned") pinned();
+    else if (what == "together") together();
+    else if (what == "short_of_memory") short_of_memory();
     else return 2;
     std::printf("%s ok\n", what.c_str());
     return 0;
