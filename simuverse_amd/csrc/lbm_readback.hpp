@@ -2,9 +2,10 @@
 //
 // hipMemcpyAsync into pageable memory goes through the runtime's own staging
 // on the calling thread: 10 GB/s for the 201 MB of a 4096^2 macro field (19.2
-// ms), and 0.41 ms for a single megabyte, which the link carries into pinned
-// memory in 27 us (57 GB/s for large copies).  Fresh host pages are the other
-// bound: one thread fills them at 4 GB/s where the kernel has to clear them.
+// ms), and 82 us for a single megabyte into pages that are there, which the
+// link carries into pinned memory in 27 us (57 GB/s for large copies).  Fresh
+// host pages are the other bound: one thread fills them at 4 GB/s where the
+// kernel has to clear them (300 us for that megabyte).
 //
 // Staging copies through pinned slots, which the objects on a device share.  A
 // small readback pipelines its chunks through them on the calling thread; a
@@ -185,12 +186,17 @@ private:
         size_t at, bytes;        // in the run
     };
     static constexpr size_t kSlot = SlotPool::kSlot;
-    // Below 6 MiB one thread and two slots that take turns (the link fills one
+    // Below 4 MiB one thread and two slots that take turns (the link fills one
     // faster than the thread empties the other), four threads up to 32 MiB,
-    // twelve beyond.  One thread and four, microseconds, a program's arrays
-    // reused and kept: 5.0 MB 250 to 1180 and 600 to 750; 6.7 MB 1040 to 1400
-    // and 720 to 800; 12.6 MB 1490 to 1880 and 900.
-    static constexpr size_t kThreaded = 6u << 20, kMore = 32u << 20;
+    // twelve beyond.  Microseconds through the runtime, with one thread and
+    // with four, into pages that are there / that the kernel has to clear:
+    //   1.80 MB  115 / 480   95 / 450  114 / 300   5.88 MB 347 / 1570  285 / 1480  268 / 1060
+    //   3.15 MB  205 / 880  160 / 825  171 / 628   7.08 MB 450 / 1950   -          320 / 1250
+    //   4.32 MB  285 / 1260 224 / 1106 235 / 775  12.58 MB 770 / 3430   -          500 / 2120
+    // A page's state is not known here: the line lies where four threads cost
+    // nothing into pages that are there (3.15 MB: 7 %; from 4.3 MB on within
+    // the scatter), because they save a quarter and more into the others.
+    static constexpr size_t kThreaded = 4u << 20, kMore = 32u << 20;
     static constexpr size_t slots_for(size_t total)
     {
         return total < kThreaded ? 2 : (total < kMore ? 4 : SlotPool::kSlots);

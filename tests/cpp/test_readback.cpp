@@ -57,7 +57,7 @@ static void bytes()
 {
     fake::Stream s;
     Staging st;
-    for (size_t n : {4ul, 36ul, 350000ul, MiB, MiB + 4, 2 * MiB - 4, 2 * MiB + 8, 7 * MiB + 12, 11 * MiB, 17 * MiB})
+    for (size_t n : {4ul, 36ul, 350000ul, MiB, MiB + 4, 4 * MiB / 3, 4 * MiB / 3 / 4 * 4 + 4, 2 * MiB - 4, 2 * MiB + 8, 7 * MiB + 12, 11 * MiB})
         for (bool skip : {false, true}) reads(st, &s, n, skip);
     reads(st, &s, 4, false);
 }
@@ -88,7 +88,7 @@ static void copy_fails()
 {
     fake::Stream s;
     Staging st;
-    for (size_t n : {MiB, 3 * MiB, 14 * MiB})
+    for (size_t n : {MiB, 2 * MiB, 11 * MiB})
         for (int left : {0, 1, 2}) {
             fake::copies_left = left;
             reads(st, &s, n, false, hipErrorUnknown);
@@ -111,8 +111,8 @@ static void pinned()
         CHECK(fake::pinned <= MiB);
         for (auto& st : many) reads(*st, &s, 100000, false);
         CHECK(fake::pinned <= 2 * MiB);
-        reads(*many[3], &s, 14 * MiB, false);
-        reads(*many[4], &s, 14 * MiB, false);
+        reads(*many[3], &s, 11 * MiB, false);
+        reads(*many[4], &s, 11 * MiB, false);
         CHECK(fake::pinned <= 12 * MiB);
         while (many.size() > 1) many.pop_back();
         reads(*many[0], &s, 3 * MiB, true);
@@ -151,7 +151,7 @@ static void together()
 static void short_of_memory()
 {
     fake::Stream s;
-    for (size_t n : {1000ul, MiB, 3 * MiB, 14 * MiB})
+    for (size_t n : {1000ul, MiB, 2 * MiB})
         for (int good : {0, 1, 5}) {
             Staging st;
             if (good) reads(st, &s, (good == 1 ? 1 : 4) * MiB / 4, false);
