@@ -771,6 +771,7 @@ int mlp_grad(lbm_mlp* m, const float* X, const float* T, int n, int batch, uint6
         if (m->loss_part) (void)hipFree(m->loss_part);
         m->partial = nullptr;
         m->loss_part = nullptr;
+        m->partial_blocks = 0;  // until both are there
         MLP_TRY(hipMalloc(&m->partial, (size_t)nb * kMlpParams * sizeof(float)));
         MLP_TRY(hipMalloc(&m->loss_part, (size_t)nb * sizeof(double)));
         m->partial_blocks = nb;
