@@ -86,7 +86,7 @@ struct lbm_handle {
     float omega = 1.0f;
     float scale = 1.0f, inv_scale = 1.0f;
     int variant = 6;
-    bool auto_shape = true;  // no shape chosen by the caller: lbm_run takes default_shape's
+    bool auto_shape = true;  // no shape chosen by the caller: lbm_run takes default_step_variant's
     int graph_chunk = 100;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -176,8 +176,6 @@ hipError_t enqueue_step(lbm_handle* h, int swap, bool export_macro)
                             h->macro, h->stream);
 }
 
-// Steps one launch advances: 2 or 3 for a multi-step variant on a plain
-// physics handle, else 1.
 // The shape lbm_run steps with: the caller's (lbm_set_variant, lbm_autotune),
 // else the one the lattice's size asks for.
 int run_variant(const lbm_handle* h)
@@ -185,6 +183,8 @@ int run_variant(const lbm_handle* h)
     return h->auto_shape ? default_step_variant(h->f16, h->d.nx, h->d.ny, h->d.x_edge, h->variant) : h->variant;
 }
 
+// Steps one launch advances: a multi-step variant's number on a plain physics
+// handle, else 1.
 int launch_steps(const lbm_handle* h) { return h->physics() && !h->mlp ? step_variant_steps(run_variant(h)) : 1; }
 
 // Steps at the end of a run that take one-step launches whatever is left

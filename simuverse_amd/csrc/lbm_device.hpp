@@ -438,10 +438,6 @@ constexpr int kOffB3 = kOffW3 + kMlpOut * kMlpH;
 constexpr int kMlpParams = kOffB3 + kMlpOut;  // 5385
 
 __device__ inline float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ inline float gelu_grad(float x)
-{
-    return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * expf(-0.5f * x * x) * 0.39894228040143268f;
-}
 
 // The network on one sample in binary32; P holds the parameter vector
 // (in LDS in the kernels that call this).

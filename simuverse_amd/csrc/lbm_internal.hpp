@@ -46,7 +46,7 @@ inline int step_variant_steps(int variant)
 }
 // Whether two-step tiles of width bw fit an nx x ny lattice (lbm_step2.hip).
 bool two_step_fits(int bw, int nx, int ny, int xedge);
-// Whether ns-step tiles of width bw fit (lbm_stepn.hip): the two-step rule,
+// Whether ns-step tiles (lbm_stepn.hip) of width bw fit: the two-step rule,
 // and a ring of ns - 1 cells that wraps around the lattice at most once.
 inline bool nstep_fits(int bw, int ns, int nx, int ny, int xedge)
 {
