@@ -81,11 +81,16 @@ struct Stream {
 };
 inline std::atomic<size_t> pinned{0}, pinned_most{0}, events{0};
 inline std::atomic<int> waiting{0};      // threads inside a wait of the runtime
+inline std::atomic<int> waits{0}, records{0};  // calls so far
 inline std::atomic<int> fail_pin{0};     // this many pinned allocations fail
 inline std::atomic<int> fail_event{0};
 inline std::atomic<int> copies_left{-1};  // copies until one fails, -1: none does
 struct Wait {
-    Wait() { ++waiting; }
+    Wait()
+    {
+        ++waiting;
+        ++waits;
+    }
     ~Wait() { --waiting; }
 };
 }  // namespace fake
@@ -138,6 +143,7 @@ inline hipError_t hipEventDestroy(hipEvent_t e)
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 {
     size_t at;
+    ++fake::records;
     {
         std::lock_guard<std::mutex> l(e->mu);
         at = ++e->recorded;

@@ -62,6 +62,22 @@ static void bytes()
     reads(st, &s, 4, false);
 }
 
+// A readback of one chunk makes one copy and one wait, no event: what the
+// runtime's own copy costs a small frame.
+static void one_chunk()
+{
+    fake::Stream s;
+    Staging st;
+    for (size_t n : {8ul, 40000ul, MiB / 3}) {
+        fake::waits = fake::records = 0;
+        reads(st, &s, n, false);
+        CHECK(fake::waits == 1 && fake::records == 0);
+    }
+    fake::waits = fake::records = 0;
+    reads(st, &s, MiB, false);  // three chunks
+    CHECK(fake::waits == 3 && fake::records == 2);
+}
+
 // While the stream has other work before the readback, only the calling thread
 // waits inside the runtime, whose waits spin.
 static void busy()
@@ -170,6 +186,7 @@ int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") bytes();
+    else if (what == "one_chunk") one_chunk();
     else if (what == "busy") busy();
     else if (what == "copy_fails") copy_fails();
     else if (what == "pinned") pinned();

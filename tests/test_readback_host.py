@@ -22,7 +22,7 @@ def program(request, tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["bytes", "busy", "copy_fails", "pinned", "together", "short_of_memory"])
+@pytest.mark.parametrize("what", ["bytes", "one_chunk", "busy", "copy_fails", "pinned", "together", "short_of_memory"])
 def test_readback(program, what):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1", TSAN_OPTIONS="halt_on_error=1")
     r = subprocess.run([str(program), what], capture_output=True, text=True, timeout=120, env=env)
