@@ -246,13 +246,15 @@ __global__ __launch_bounds__(BS) void k3_step(Args3 a, const T* __restrict__ src
 // bit for bit at every slot a fluid cell can read.
 //
 // The one-step kernel is bound by HBM (152 B per cell and step in binary32);
-// here two steps share one read, with the ring's, and one write, and what
-// bounds it is each turn's chain (loads a turn ahead, collision, barrier,
-// pulls, collision, stores) with 16 wavefronts on a CU.  The autotuner takes
-// it in binary32 at middle sizes, microseconds per step for the best one-step
-// shape and the two of these: 100x90x80 23.5, 17.7, 17.6; 200x144x90 75.0,
-// 68.2, 63.7; 256x60x200 79.9, 77.1, 88.8; 256^3 453.5, 454.9, 525.7.  In
-// binary16 the one-step shapes stay ahead.
+// here two steps share one read, with the ring's, and one write (at 256^3 3.70
+// GB per launch, 0.72 of two one-step launches), and what bounds it is each
+// turn's chain (loads a turn ahead, collision, barrier, pulls, collision,
+// stores): of 3.3 wavefronts per SIMD one issues a quarter of the time.  The
+// autotuner takes it in binary32 at middle sizes, microseconds per step for the
+// best one-step shape and the two of these, with force from rest: 100x90x80
+// 22.2, 16.1, 16.8; 200x144x90 71.7, 64.0, 62.7; 256x60x200 76.6, 73.2, 86.1;
+// 256^3 419, 438, 520 (with spheres and a flow 454, 455, 526).  In binary16 the
+// one-step shapes stay ahead.
 constexpr int side_slot(int i)  // place of a sideways direction among those of its ez
 {
     int n = 0;

@@ -134,17 +134,20 @@ __global__ __launch_bounds__(256) void k_mlp_forward_mma(const E* __restrict__ p
 // outputs use the 4x4x1 form: block l / 4 holds four samples, the two lane
 // halves sum different units and are added at the end.
 //
-// What bounds it: 16 384 matrix-core cycles per 32 samples and SIMD and
-// about as many of vector instructions (64 erf and exp pairs per lane);
-// two wavefronts per SIMD overlap the two.  Each wavefront keeps its sums
-// of the gradient (105 registers) across its chunks, so memory sees each
-// sample once and one partial per block.  Measured on 10^6 samples: 0.40 ms
-// (75 TFLOP/s of the 154 a large binary32 matrix product reaches; matrix
-// cores busy 55 %, vector ALUs 25 %), against 2.25 ms for the same sums on
-// the vector ALUs with activations staged in LDS; 4096 samples: 25 us
-// against 40 us.  Gradient error against binary64 at 4096 samples 4e-8
-// (1.1e-7 before: the partials of at most 256 blocks are now added in
-// binary64).
+// What bounds it: 16 384 matrix-core cycles per 32 samples and SIMD, 54 % of
+// the launch, and the chain around them: the vector instructions (64 GELU and
+// derivative pairs per lane) issue for 12 to 14 % and the LDS is busy for 13 %,
+// but two wavefronts per SIMD overlap the phases only in part and wait for a
+// third of their time.  Each wavefront keeps its sums of the gradient (105
+// registers) across its chunks, so memory sees each sample once and one partial
+// per block.  All 256 registers are used and 27 values go through scratch
+// memory, most of them stored once before the loop over chunks; every store of
+// one runs with all lanes on.  Measured on 10^6 samples: 0.40 ms (75 TFLOP/s of
+// the 154 a large binary32 matrix product reaches), against 2.25 ms for the
+// same sums on the vector ALUs with activations staged in LDS; 4096 samples: 25
+// us against 40 us.  Gradient error against binary64 at 4096 samples 3.5e-8
+// (1.2e-7 before: the partials of at most 256 blocks are now added in
+// binary64); for single samples 2.6e-7 (2.8e-7).
 // ---------------------------------------------------------------------------
 constexpr int kTS = 32;             // samples a wavefront takes at a time
 constexpr int kGradWaves = 8;       // wavefronts per block (two per SIMD)
@@ -179,9 +182,9 @@ inline int mlp_grad_blocks(int batch) { return std::min((batch + kTS - 1) / kTS,
 //   1 - Phi(|x|) = e (c1 t + c2 t^2 + .. + c7 t^7)
 // (the form of Abramowitz & Stegun 7.1.26; coefficients fitted to
 // erfcx(|x| / sqrt 2) / 2 by reweighted least squares, largest deviation of
-// Phi 2e-9 before rounding).  Evaluated in binary32 over [-9, 9] against
-// binary64: GELU rms 5.7e-8 (largest 3.8e-7, at |x| near 9), derivative rms
-// 2.4e-8, as the erff form (6.4e-8, 4.5e-7, 2.4e-8).  No branch: 17 vector
+// Phi 8.3e-9 before rounding, at |x| = 0.38).  On the device over [-9, 9]
+// against binary64: GELU rms 5.6e-8 (largest 3.7e-7, at |x| near 9), derivative
+// rms 2.6e-8, as the erff form (6.4e-8, 4.5e-7, 2.4e-8).  No branch: 17 vector
 // instructions, where erff and expf take about 80 with both sides of erff's
 // branch.
 __device__ __forceinline__ void gelu_both(float x, float& y, float& d)

@@ -23,18 +23,24 @@ namespace lbm {
 // one-step launches leave it (at every slot a fluid cell can read); NS is
 // odd, so also in the same buffer.
 //
-// Bound by its vector instructions (HBM moves one read and one write of the
-// state per NS steps): with the masks read once, addresses that a step only
-// reads with constant offsets and the step loop unrolled, a pass of 64 cells
-// takes 83 of them in binary32 with force between LDS and LDS, where the
-// three-step tile takes 128.  That is what makes the wider ring of five
-// steps pay: 4096^2 binary32 periodic with force 72 us per step against 90
+// What bounds it: in binary32 no unit alone.  At 4096^2 the SIMDs issue vector
+// instructions for about half of a launch (binary32 arithmetic and 32-bit
+// logic take two cycles of a SIMD, shifts, compares, selects and conversions
+// four), the LDS is busy for 26 % without bank conflicts, HBM carries one read
+// and one write of the state per NS steps (1.40 GB, 3.6 TB/s), and wavefronts
+// wait for half of their time on the chain of loads, collision and barriers.
+// In binary16 the conversions bring the issue to two thirds to three quarters.
+// Fewer instructions shorten both the chain and the issue: with the masks read
+// once, addresses that a step only reads with constant offsets and the step
+// loop unrolled, a pass of 64 cells takes 83 of them in binary32 with force
+// between LDS and LDS, where the three-step tile takes 128.  That is what makes
+// the wider ring of five steps pay: 4096^2 binary32 periodic with force 72 us per step against 90
 // for the three-step 64 x 24 tile, 8192^2 binary16 253 (64 x 48 region)
 // against 281.  On small lattices the launches count instead (a launch of a
 // few blocks takes about 3 us, however little it computes): 256^2 1.3 us per
 // step with nine steps per launch against 3.8 with one.  A step loop left
 // rolled keeps the registers of every step live and spills with two cells
-// per thread; seven steps on the 64 x 32 region lose more to the ring than
+// per thread (the build refuses that); seven steps on the 64 x 32 region lose more to the ring than
 // they save (74 against 72 us), and binary32 regions of 64 x 48 leave one
 // block per CU (95).
 enum : uint32_t {

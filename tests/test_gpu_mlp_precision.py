@@ -36,7 +36,7 @@ def gelu_at(net, a):
 
 
 def test_gelu_and_its_derivative():
-    """Bounds: with q = 1 - Phi(|x|), the fit is off by 8e-9 at most; q carries
+    """Bounds: with q = 1 - Phi(|x|), the fit is off by 8.3e-9 at most; q carries
     the roundings of a reciprocal, seven polynomial steps, two products and an
     exponential (14 units of 2^-24) and x^2 units from the exponent's argument;
     1 - q rounds once; then x Phi, or the product x phi(x) and its sum, and the
@@ -52,7 +52,7 @@ def test_gelu_and_its_derivative():
     q = 0.5 * erfc
     Phi = np.where(X >= 0, 1.0 - q, q)
     dens = np.exp(-0.5 * X * X) / math.sqrt(2.0 * math.pi)
-    dPhi = 8e-9 + q * (14 + X * X) * U + U
+    dPhi = 8.3e-9 + q * (14 + X * X) * U + U
     ey, ed = np.abs(y - X * Phi), np.abs(d - (Phi + X * dens))
     print(f"  GELU error: largest {ey.max():.2e}, rms {np.sqrt((ey**2).mean()):.2e}; derivative: largest {ed.max():.2e}, "
           f"rms {np.sqrt((ed**2).mean()):.2e}", flush=True)
