@@ -284,7 +284,8 @@ private:
         const size_t hw = std::max(1u, std::thread::hardware_concurrency());
         const size_t workers = std::min({slots.count, n, hw});
         std::atomic<int> error{(int)hipSuccess};
-        std::atomic<size_t> next{1};  // chunk 0 is the calling thread's
+        std::atomic<size_t> next{0};
+        size_t issued = 0;  // chunk w is worker w's first, on its way before the worker wakes
         std::mutex gate;
         std::condition_variable opened;
         bool open = false;
@@ -300,17 +301,25 @@ private:
                 std::unique_lock<std::mutex> lock(gate);
                 opened.wait(lock, [&] { return open; });
             }
-            rest(w, hipSetDevice(dev));
+            hipError_t e = hipSetDevice(dev);
+            if (e == hipSuccess && w < issued) e = take(chunks[w], *slots.slot[w]);
+            rest(w, e);
         };
         std::vector<std::thread> threads;
         hipError_t e = issue(chunks[0], *slots.slot[0], s);
+        if (e == hipSuccess) issued = 1;
         try {
             threads.reserve(workers);
-            for (size_t w = 1; w < workers; ++w) threads.emplace_back(work, w);
+            while (e == hipSuccess && issued < workers) {
+                threads.emplace_back(work, issued);
+                e = issue(chunks[issued], *slots.slot[issued], s);
+                if (e == hipSuccess) ++issued;
+            }
         } catch (...) {  // no thread to be had: the ones that started, and this one, do the work
         }
         if (e == hipSuccess) e = hipEventSynchronize(slots.slot[0]->event);
         if (e != hipSuccess) error.store((int)e);
+        next.store(issued);
         {
             std::lock_guard<std::mutex> lock(gate);
             open = true;
